@@ -47,6 +47,27 @@ def test_quant_bit_exact(rows, cols, nova7, oracle):
     assert np.array_equal(s.numpy((rows, cols // 16), np.int32), rs)
 
 
+@pytest.mark.parametrize("rows,cols", [(1, 32), (1, 96), (5, 160), (7, 1056), (33, 992)])
+def test_quant_partial_workgroups(rows, cols, nova7, oracle):
+    """Blocks that do not fill a wave or a workgroup (8 lanes per block), rows
+    whose blocks straddle waves, and nothing written past the last block."""
+    nova = nova7
+    print(f"[case] quant partial rows={rows} cols={cols}", flush=True)
+    rng = np.random.default_rng(rows * 31 + cols)
+    x = (rng.standard_normal((rows, cols)) * rng.uniform(1e-3, 50, (rows, 1))).astype(np.float32)
+    x[-1, -32:] = 0.0
+    n = rows * cols
+    dx = nova.upload(x)
+    qs, d, s = (nova.upload(np.full(b + 64, 0x5A, np.uint8)) for b in (n, n // 8, n // 4))
+    nova.launch_quant_q8(qs.ptr, d.ptr, s.ptr, dx.ptr, rows, cols, None)
+    nova.dev_sync()
+    rq, rd, rs = oracle.quant_q8(x)
+    for buf, ref in ((qs, rq), (d, rd), (s, rs)):
+        got = buf.numpy((ref.nbytes + 64,), np.uint8)
+        assert np.array_equal(got[:ref.nbytes], np.ascontiguousarray(ref).view(np.uint8).ravel())
+        assert np.all(got[ref.nbytes:] == 0x5A)
+
+
 @pytest.mark.parametrize("rows,cols", [(37, 256), (20, 1536), (512, 3584), (3584, 3584), (50, 5120), (11, 8192),
                                        (70, 8960), (33, 13824), (130, 18944), (9, 32768), (1000, 2560),
                                        (1, 3584), (3, 18944)])
