@@ -10,22 +10,24 @@
 //   w . x = sum over sub-blocks of dx * (d*sc*sum(q*c) - dmin*m*sum(c)).
 //
 // gfx950 design (HBM-bound on the weights, 4.5 bits each):
-//  * A workgroup of 4 waves stages the whole activation (codes, scales, sums)
-//    in LDS once and then walks rows (grid-stride), one row per wave at a
-//    time, so the activation is read from L2 once per workgroup, not per row.
-//  * One token: a wave covers 16 super-blocks per step: lane (j, c) =
-//    (lane >> 2, lane & 3) takes the 32 nibble bytes at offset 32c of
-//    super-block 16s + j -- all 32 weights of sub-block 2c (low nibbles) and
-//    of 2c+1 (high).  (The four-token kernel uses half-width lanes, 8
-//    super-blocks per step.)  Rows of up to 4 steps (cols <= 16384: the
-//    hidden widths 1536, 3584, 5120) are one wave's, with the step loop unrolled at compile time and
-//    all of a row's loads issued before any is consumed; wider rows (the FFN
-//    widths) are shared by the 4 waves of a workgroup, at most 4 steps each,
-//    reduced through LDS in a fixed order.  Grids are sized to what is
-//    resident at once and grid-stride beyond.
-//  * Products: v_dot4_i32_i8 on nibbles unpacked with a mask and a shift
-//    (8 per lane per super-block); the per-sub-block float combination is the
-//    reference's; the row sum is a wave reduction.
+//  * One token: a workgroup of 4 waves stages the whole activation (codes,
+//    scales, sums) in LDS once and then walks rows (grid-stride), so the
+//    activation is read from L2 once per workgroup, not per row.  A wave covers
+//    16 super-blocks per step: lane (j, c) = (lane >> 2, lane & 3) takes the 32
+//    nibble bytes at offset 32c of super-block 16s + j -- all 32 weights of
+//    sub-block 2c (low nibbles) and of 2c+1 (high).  Rows of up to 4 steps
+//    (cols <= 16384: the hidden widths 1536, 3584, 5120) are one wave's, with
+//    the step loop unrolled at compile time and all of a row's loads issued
+//    before any is consumed; wider rows (the FFN widths) are shared by the 4
+//    waves of a workgroup, at most 4 steps each, reduced through LDS in a fixed
+//    order.  Grids are sized to what is resident at once and grid-stride
+//    beyond.  Products: v_dot4_i32_i8 on nibbles unpacked with a mask and a
+//    shift; the per-sub-block float combination is the reference's; the row sum
+//    is a wave reduction.  The large launches run at what HBM gives them:
+//    37888 x 3584 with ActQ8 16.25 us, 152064 x 3584 57 us (5.4 TB/s); the same
+//    products from registers alone, or with the weights through LDS rings filled
+//    by direct loads (per workgroup or per wave), measured 16.0-16.5 and 55-57.
+//  * Four tokens: int8 MFMA, see gemv4_kernel.
 #include <hip/hip_runtime.h>
 #include <cstdint>
 #include <mutex>
@@ -46,25 +48,15 @@ constexpr int kQK = 256;                       // weights per super-block
 constexpr int kBlockBytes = 144;
 constexpr int QT = 256;                        // threads per workgroup
 constexpr int kMaxCols = 32768;                // the activation (and its scales, sums) fits LDS
-// Lane geometry, LPS = lanes per super-block.  LPS = 4 (one token): a lane
-// owns the 32 nibble bytes of one sub-block pair (64 weights: sub-block 2c in
-// the low nibbles, 2c+1 in the high), 16 super-blocks per wave step.  LPS = 8
-// (four tokens): half of that, 8 super-blocks per step.  Measured: the wide
-// lanes take a 7B layer's projections from 50.8 to 48.7 us (fewer, larger
-// steps per row), but make the four-token kernel 11% slower.
-template <int LPS>
-struct Lanes {
-    static_assert(LPS == 4 || LPS == 8, "4 or 8 lanes per super-block");
-    static constexpr int kSbPerStep = 64 / LPS;
-    static constexpr int kNibWords = 32 / LPS;   // nibble dwords per lane
-    static constexpr int grp(int c) { return LPS == 4 ? c : c >> 1; }
-    static constexpr int elo(int c) { return LPS == 4 ? 64 * c : (c >> 1) * 64 + (c & 1) * 16; }
-};
-constexpr int kLps1 = 4;                       // one-token kernels
-constexpr int kLps4 = 8;                       // four-token kernel
-template <int LPS>
+// One-token lane geometry: 4 lanes per super-block, each with the 32 nibble
+// bytes of one sub-block pair (64 weights: sub-block 2c in the low nibbles,
+// 2c+1 in the high), 16 super-blocks per wave step.  (8 lanes of half that
+// width: a 7B layer's projections 50.8 us against 48.7: more, smaller steps.)
+constexpr int kLps = 4;
+constexpr int kSbPerStep = 64 / kLps;
+constexpr int kNibWords = 32 / kLps;           // nibble dwords per lane
 struct Nib {
-    uint32_t w[Lanes<LPS>::kNibWords];
+    uint32_t w[kNibWords];
 };
 
 // ---------------------------------------------------------------- quant
@@ -165,26 +157,11 @@ __device__ __forceinline__ void scale_min(int j, const uint32_t sw[3], uint32_t&
     }
 }
 
-// One lane's share of a super-block, split in two so that several
-// activations can reuse one weight load: sb_prep unpacks the lane's 16 nibble
-// bytes (16 weights of sub-block 2grp in the low nibbles, 16 of 2grp+1 in the
-// high) and the two (d*scale, dmin*min) pairs; sb_dot takes the products with
-// one activation staged in LDS (codes, scales per 32, sums per 16).  The
-// float combination is the reference's: dx * (d*sc*sum(q*c) - dmin*m*sum(c)).
-template <int LPS>
-struct SbW {
-    static constexpr int NW = Lanes<LPS>::kNibWords;
-    int lo[NW], hi[NW];                // nibbles as int8 lanes for v_dot4_i32_i8
-    float al, bl, ah, bh;              // d*sc and dmin*m of the two sub-blocks
-};
-
-template <int LPS>
-__device__ __forceinline__ Nib<LPS> load_nib(const uint8_t* blk, int c) {
-    constexpr int NW = Lanes<LPS>::kNibWords;
-    Nib<LPS> n;
-    const uint8_t* p = blk + 16 + 4 * NW * c;
+__device__ __forceinline__ Nib load_nib(const uint8_t* blk, int c) {
+    Nib n;
+    const uint8_t* p = blk + 16 + 4 * kNibWords * c;
 #pragma unroll
-    for (int h = 0; h < NW / 4; ++h) {
+    for (int h = 0; h < kNibWords / 4; ++h) {
         const u4 v = *reinterpret_cast<const u4*>(p + 16 * h);
 #pragma unroll
         for (int e = 0; e < 4; ++e) n.w[4 * h + e] = v[e];
@@ -192,18 +169,29 @@ __device__ __forceinline__ Nib<LPS> load_nib(const uint8_t* blk, int c) {
     return n;
 }
 
-template <int LPS>
-__device__ __forceinline__ SbW<LPS> sb_prep(const u4 hd, const Nib<LPS>& nb, int grp) {
-    SbW<LPS> w;
+// Lane c's share of a super-block: its nibbles as int8 lanes of
+// v_dot4_i32_i8 (sub-block 2c low, 2c+1 high) and the two (d*scale, dmin*min)
+// pairs, unpacked ahead of the products with the activation staged in LDS
+// (codes, scales per 32, sums per 16).  (As one function the loads of a row's
+// later steps end up behind the earlier steps' arithmetic: a 5120-wide layer
+// 3% slower.)  The float combination is the reference's:
+// dx * (d*sc*sum(q*c) - dmin*m*sum(c)).
+struct SbW {
+    int lo[kNibWords], hi[kNibWords];
+    float al, bl, ah, bh;
+};
+
+__device__ __forceinline__ SbW sb_prep(const u4 hd, const Nib& nb, int c) {
+    SbW w;
 #pragma unroll
-    for (int e = 0; e < SbW<LPS>::NW; ++e) {
+    for (int e = 0; e < kNibWords; ++e) {
         w.lo[e] = (int)(nb.w[e] & 0x0F0F0F0Fu);
         w.hi[e] = (int)((nb.w[e] >> 4) & 0x0F0F0F0Fu);
     }
     const uint32_t sw[3] = {hd[1], hd[2], hd[3]};
     uint32_t scl, mcl, sch, mch;
-    scale_min(2 * grp, sw, scl, mcl);
-    scale_min(2 * grp + 1, sw, sch, mch);
+    scale_min(2 * c, sw, scl, mcl);
+    scale_min(2 * c + 1, sw, sch, mch);
     const float dd = half_to_float(hd[0] & 0xFFFFu);
     const float dm = half_to_float(hd[0] >> 16);
     w.al = dd * (float)scl;
@@ -214,13 +202,10 @@ __device__ __forceinline__ SbW<LPS> sb_prep(const u4 hd, const Nib<LPS>& nb, int
 }
 
 // k0: the lane's first element (low nibbles) in the row; high nibbles at k0 + 32
-template <int LPS>
-__device__ __forceinline__ float sb_dot(const SbW<LPS>& w, int k0, const int8_t* s_q, const float* s_d,
-                                        const float* s_s) {
-    constexpr int NW = SbW<LPS>::NW;
+__device__ __forceinline__ float sb_dot(const SbW& w, int k0, const int8_t* s_q, const float* s_d, const float* s_s) {
     int dlo = 0, dhi = 0;
 #pragma unroll
-    for (int h = 0; h < NW / 4; ++h) {
+    for (int h = 0; h < kNibWords / 4; ++h) {
         const i4 alo = *reinterpret_cast<const i4*>(s_q + k0 + 16 * h);
         const i4 ahi = *reinterpret_cast<const i4*>(s_q + k0 + 32 + 16 * h);
 #pragma unroll
@@ -231,17 +216,14 @@ __device__ __forceinline__ float sb_dot(const SbW<LPS>& w, int k0, const int8_t*
     }
     const float dxl = s_d[k0 >> 5], dxh = s_d[(k0 + 32) >> 5];
     float sml = s_s[k0 >> 4], smh = s_s[(k0 + 32) >> 4];
-    if constexpr (NW == 8) {                   // 32 elements: both 16-sums
-        sml += s_s[(k0 >> 4) + 1];
-        smh += s_s[((k0 + 32) >> 4) + 1];
-    }
+    sml += s_s[(k0 >> 4) + 1];
+    smh += s_s[((k0 + 32) >> 4) + 1];
     return dxl * (w.al * (float)dlo - w.bl * sml) + dxh * (w.ah * (float)dhi - w.bh * smh);
 }
 
-template <int LPS>
-__device__ __forceinline__ float sb_terms(const u4 hd, const Nib<LPS>& nb, int sb, int grp, int elo,
-                                          const int8_t* s_q, const float* s_d, const float* s_s) {
-    return sb_dot<LPS>(sb_prep<LPS>(hd, nb, grp), sb * kQK + elo, s_q, s_d, s_s);
+__device__ __forceinline__ float sb_terms(const u4 hd, const Nib& nb, int sb, int c, int elo, const int8_t* s_q,
+                                          const float* s_d, const float* s_s) {
+    return sb_dot(sb_prep(hd, nb, c), sb * kQK + elo, s_q, s_d, s_s);
 }
 
 // Up to 4 matrices of the same width that read one activation (q/k/v,
@@ -339,19 +321,17 @@ __device__ __forceinline__ void stage_activation(const GemvSet& g, int8_t* s_q, 
 // keeps more bytes in flight per wave but costs occupancy and is slower.)
 template <int STEPS, bool kF32>
 __global__ void __launch_bounds__(QT) gemv_fixed_kernel(GemvSet g) {
-    constexpr int LPS_ = kLps1;
     extern __shared__ __attribute__((aligned(16))) unsigned char s_x[];
     const int cols = g.cols;
     int8_t* s_q = reinterpret_cast<int8_t*>(s_x);
     float* s_d = reinterpret_cast<float*>(s_x + cols);
     float* s_s = reinterpret_cast<float*>(s_x + cols + 4 * (cols / 32));   // 16-sums as exact floats
-    stage_activation<kF32, STEPS * Lanes<kLps1>::kSbPerStep * kQK>(g, s_q, s_d, s_s);
+    stage_activation<kF32, STEPS * kSbPerStep * kQK>(g, s_q, s_d, s_s);
 
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // wave-uniform: scalar row addressing
-    using L = Lanes<LPS_>;
-    const int j = lane / LPS_, c = lane % LPS_, grp = L::grp(c);
-    const int elo = L::elo(c);
+    const int j = lane / kLps, c = lane % kLps;
+    const int elo = 64 * c;
     const int nsb = cols / kQK;
     const int64_t row_bytes = (int64_t)nsb * kBlockBytes;
     const int64_t rows = kF32 ? g.end[g.n - 1] : g.end[0];   // one matrix on the ActQ8 path
@@ -361,21 +341,21 @@ __global__ void __launch_bounds__(QT) gemv_fixed_kernel(GemvSet g) {
         const int64_t lr = m ? r - g.end[m - 1] : r;
         const uint8_t* wr = g.w[m] + lr * row_bytes;
         u4 hdr[STEPS];
-        Nib<LPS_> nib[STEPS];
+        Nib nib[STEPS];
 #pragma unroll
         for (int t = 0; t < STEPS; ++t) {
-            const int sb = L::kSbPerStep * t + j;
+            const int sb = kSbPerStep * t + j;
             if (sb < nsb) {
                 const uint8_t* blk = wr + (int64_t)sb * kBlockBytes;
                 hdr[t] = *reinterpret_cast<const u4*>(blk);
-                nib[t] = load_nib<LPS_>(blk, c);
+                nib[t] = load_nib(blk, c);
             }
         }
         float acc = 0.f;
 #pragma unroll
         for (int t = 0; t < STEPS; ++t) {
-            const int sb = L::kSbPerStep * t + j;
-            if (sb < nsb) acc += sb_terms<LPS_>(hdr[t], nib[t], sb, grp, elo, s_q, s_d, s_s);
+            const int sb = kSbPerStep * t + j;
+            if (sb < nsb) acc += sb_terms(hdr[t], nib[t], sb, c, elo, s_q, s_d, s_s);
         }
 #pragma unroll
         for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o, 64);
@@ -389,24 +369,22 @@ __global__ void __launch_bounds__(QT) gemv_fixed_kernel(GemvSet g) {
 // iteration.
 template <int STEPS, int KS, bool kF32>
 __global__ void __launch_bounds__(QT) gemv_split_kernel(GemvSet g) {
-    constexpr int LPS_ = kLps1;
     extern __shared__ __attribute__((aligned(16))) unsigned char s_x[];
     __shared__ float s_part[4];
     const int cols = g.cols;
     int8_t* s_q = reinterpret_cast<int8_t*>(s_x);
     float* s_d = reinterpret_cast<float*>(s_x + cols);
     float* s_s = reinterpret_cast<float*>(s_x + cols + 4 * (cols / 32));   // 16-sums as exact floats
-    stage_activation<kF32, (STEPS * Lanes<kLps1>::kSbPerStep * kQK * KS < kMaxCols ? STEPS * Lanes<kLps1>::kSbPerStep * kQK * KS : kMaxCols)>(g, s_q, s_d, s_s);
+    stage_activation<kF32, (STEPS * kSbPerStep * kQK * KS < kMaxCols ? STEPS * kSbPerStep * kQK * KS : kMaxCols)>(g, s_q, s_d, s_s);
 
     constexpr int RPI = 4 / KS;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // wave-uniform: scalar row addressing
     const int part = wave % KS;
-    using L = Lanes<LPS_>;
-    const int j = lane / LPS_, c = lane % LPS_, grp = L::grp(c);
-    const int elo = L::elo(c);
+    const int j = lane / kLps, c = lane % kLps;
+    const int elo = 64 * c;
     const int nsb = cols / kQK;
-    const int sb0 = L::kSbPerStep * STEPS * part + j;
+    const int sb0 = kSbPerStep * STEPS * part + j;
     const int64_t row_bytes = (int64_t)nsb * kBlockBytes;
     const int64_t rows = kF32 ? g.end[g.n - 1] : g.end[0];   // one matrix on the ActQ8 path
     const int64_t stride = (int64_t)gridDim.x * RPI;
@@ -419,20 +397,20 @@ __global__ void __launch_bounds__(QT) gemv_split_kernel(GemvSet g) {
         if (r < rows) {
             const uint8_t* wr = g.w[m] + lr * row_bytes;
             u4 hdr[STEPS];
-            Nib<LPS_> nib[STEPS];
+            Nib nib[STEPS];
 #pragma unroll
             for (int t = 0; t < STEPS; ++t) {
-                const int sb = sb0 + L::kSbPerStep * t;
+                const int sb = sb0 + kSbPerStep * t;
                 if (sb < nsb) {
                     const uint8_t* blk = wr + (int64_t)sb * kBlockBytes;
                     hdr[t] = *reinterpret_cast<const u4*>(blk);
-                    nib[t] = load_nib<LPS_>(blk, c);
+                    nib[t] = load_nib(blk, c);
                 }
             }
 #pragma unroll
             for (int t = 0; t < STEPS; ++t) {
-                const int sb = sb0 + L::kSbPerStep * t;
-                if (sb < nsb) acc += sb_terms<LPS_>(hdr[t], nib[t], sb, grp, elo, s_q, s_d, s_s);
+                const int sb = sb0 + kSbPerStep * t;
+                if (sb < nsb) acc += sb_terms(hdr[t], nib[t], sb, c, elo, s_q, s_d, s_s);
             }
         }
 #pragma unroll
@@ -449,92 +427,234 @@ __global__ void __launch_bounds__(QT) gemv_split_kernel(GemvSet g) {
     }
 }
 
+// ---------------------------------------------------------------- direct loads
+// Direct global -> LDS loads: the wave's 64 pieces of 16 B go to the 1 KiB at
+// LDS byte address lds.  Inline asm, so that the compiler's vmcnt bookkeeping
+// does not see them (it would drain them before every LDS read it cannot prove
+// disjoint); wave_wait waits for them.  m0 cannot be declared clobbered, so the
+// statement saves and restores it.
+__device__ __forceinline__ void stream_load(const void* base, uint32_t off, uint32_t lds) {
+    // wave-uniform base: kept in scalar registers whatever the compiler made of it
+    const uint64_t b = (uint64_t)base;
+    const uint64_t sb = ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(b >> 32)) << 32) |
+                        (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)b);
+    uint32_t saved;
+    asm volatile(
+        "s_mov_b32 %0, m0\n\t"
+        "s_mov_b32 m0, %3\n\tglobal_load_lds_dwordx4 %2, %1\n\t"
+        "s_mov_b32 m0, %0"
+        : "=&s"(saved)
+        : "s"(sb), "v"(off), "s"(lds)
+        : "memory");
+}
+
+// The same with an address per lane.
+__device__ __forceinline__ void stream_load_at(const void* p, uint32_t lds) {
+    uint32_t saved;
+    asm volatile(
+        "s_mov_b32 %0, m0\n\t"
+        "s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %1, off\n\t"
+        "s_mov_b32 m0, %0"
+        : "=&s"(saved)
+        : "v"(p), "s"(lds)
+        : "memory");
+}
+
+__device__ __forceinline__ uint32_t lds_address(const unsigned char* p) {
+    return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const unsigned char*)p;
+}
+
 // Four tokens at once (the reference's gemv4_kernel, q4k_gemv.cu:98-180, as
-// Engine::decode_batch uses it for every projection, model.cpp:270-311):
-// each weight load and its scale unpacking serve four activations.  The four
-// activations (4 x 1.375 B per column) sit in LDS, 104 KB at the FFN width,
-// so a workgroup is 16 waves to keep the CU's waves up.  Lanes are half as
-// wide as in the one-token kernels (8 per super-block), so each token's sum
-// is taken in another order than launch_gemv_q4k's (same terms).
+// Engine::decode_batch uses it for every projection, model.cpp:270-311), on the
+// matrix cores: each weight is read once for the four activations.
+//
+// A unit is one super-block of 16 rows.  v_mfma_i32_16x16x64_i8 multiplies the
+// activations' codes (A) by the rows' nibbles (B): lane (g,c) reads, for each
+// half h of the super-block, row c's 16 nibble bytes at offset 16(g&1) of
+// sub-block pair 2h + (g>>1); the low nibbles are the B operand of the first
+// MFMA (sub-blocks 4h and 4h+2), the high nibbles that of the second (4h+1 and
+// 4h+3).  A's row 4j + t is token t against sub-block 4h + j: lane (g, 4j+t)
+// holds its 16 codes at 16(g&1) when j>>1 == g>>1 and zeros otherwise.  Rows
+// whose sub-block is the other MFMA's hold garbage; lane (g,c) takes the C tile
+// of MFMA g&1, whose rows 4g..4g+3 are the four tokens against sub-block 4h+g
+// of row c.  One header read and one scale decode thus serve four values of
+// the float combination dx * (d*sc*sum(q*c) - dmin*m*sum(c)); the tokens' scales
+// and sums sit in one register each (lane t of a row of 16: the scale of token
+// t, lane 4 + t: its sum) and reach the lanes as DPP row broadcasts.
+//
+// What bounds it: bytes in flight.  A unit's operands reach the wave through
+// two unit buffers of LDS that belong to it alone (the next unit is on its way
+// during this one's arithmetic): direct global -> LDS loads of 16 B pieces in
+// address order.  Loaded into registers the MFMA's way, the 16 rows put every
+// lane of a load on a line of its own: 343 cache accesses per unit (counted)
+// against ~75, and the cache's one access per clock set the pace (18944 x 3584:
+// 13.1 us against 11.6).  The activations come the same way, per unit and from
+// L2: staging all four first, as a dot4 kernel and an earlier form of this one
+// did, delays every launch by a round trip and a barrier.  No barrier holds a
+// wave to the others' pace.  Three or four buffers leave fewer waves per CU and
+// are slower (18944 x 3584: 11.7, 13.2 us; 3584 x 18944: 12.7, 13.5 against
+// 12.4); one ring per workgroup of 16 waves is faster on the largest (306 MB:
+// 60 against 75 us) and slower elsewhere (3584 x 3584: 5.7 against 4.5 us).
+// Measured against the dot4 kernel (below 32M weights) and the staged MFMA
+// kernel (above) that it replaces, us per launch: 512 x 3584 5.6 -> 4.2,
+// 3584 x 3584 6.5 -> 4.5, 18944 x 3584 14.4 -> 11.6, 3584 x 18944 16.5 -> 12.4,
+// 1536 x 1536 4.4 -> 3.4, 5120 x 13824 19.3 -> 15.7, 152064 x 3584 85 -> 75.
+// ks waves share a 16-row block's super-blocks; their sums meet in LDS and are
+// added in a fixed order.
 constexpr int kTok4 = 4;
-constexpr int QT4 = 1024;                      // threads per workgroup
-constexpr int kMaxCols4 = 28672;               // 4 activations within 160 KB of LDS
+constexpr int kMaxCols4 = 28672;
+constexpr int kMaxKs4 = 16;                    // waves of a workgroup, at most
+constexpr int kLdsMax = 160 * 1024;
+// a unit in LDS: 144 weight pieces, 8 of scales ([token][8]), 16 of sums
+// ([token][16]), 24 unused, 64 of codes ([token][256])
+constexpr int kUnitLoads = 4, kUnitBytes = 4096, kUnitX = 144 * 16, kUnitA = 3072;
 
-template <int STEPS, int KS>
-__global__ void __launch_bounds__(QT4) gemv4_kernel(const uint8_t* __restrict__ w, int64_t rows, int cols,
-                                                     const int8_t* __restrict__ xq, const float* __restrict__ xd,
-                                                     const int32_t* __restrict__ xs, float* __restrict__ out) {
-    constexpr int LPS_ = kLps4;
+// lane N of each row of 16 lanes, to the whole row
+template <int N>
+__device__ __forceinline__ float row_lane(float v) {
+    return dpp_f<0x150 + N>(v);
+}
+
+__global__ void __launch_bounds__(64 * kMaxKs4) gemv4_kernel(const uint8_t* __restrict__ w, int64_t rows, int cols,
+                                                          const int8_t* __restrict__ xq,
+                                                          const float* __restrict__ xd,
+                                                          const int32_t* __restrict__ xs, float* __restrict__ out,
+                                                          int share, int extra) {
     extern __shared__ __attribute__((aligned(16))) unsigned char s_x[];
-    __shared__ float s_part[QT4 / 64][kTok4];
-    int8_t* s_q = reinterpret_cast<int8_t*>(s_x);                                   // [4][cols]
-    float* s_d = reinterpret_cast<float*>(s_x + kTok4 * cols);                       // [4][cols/32]
-    float* s_s = reinterpret_cast<float*>(s_x + kTok4 * cols + 4 * kTok4 * (cols / 32));   // [4][cols/16]
-    stage_q8<QT4, kTok4 * kMaxCols4>(xq, xd, xs, kTok4 * cols, s_q, s_d, s_s);
-    __syncthreads();
-
-    constexpr int WAVES4 = QT4 / 64;
-    constexpr int RPI = WAVES4 / KS;           // rows per workgroup iteration
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int part = wave % KS;
-    using L = Lanes<LPS_>;
-    const int j = lane / LPS_, c = lane % LPS_, grp = L::grp(c);
-    const int elo = L::elo(c);
+    const int tid = threadIdx.x, lane = tid & 63, ks = blockDim.x >> 6;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int g = lane >> 4, c = lane & 15, t = c & 3, j = c >> 2;
     const int nsb = cols / kQK;
-    const int sb0 = L::kSbPerStep * STEPS * part + j;
-    const int64_t row_bytes = (int64_t)nsb * kBlockBytes;
-    const int64_t stride = (int64_t)gridDim.x * RPI;
+    const int sb_a = wave * nsb / ks, sb_b = (wave + 1) * nsb / ks;
+    const uint32_t row_bytes = (uint32_t)nsb * kBlockBytes;
+    // LDS: the waves' buffers | 16 zero bytes per wave | the waves' sums of two row blocks
+    unsigned char* ring = s_x + wave * (2 * kUnitBytes);
+    unsigned char* s_zero = s_x + ks * (2 * kUnitBytes) + 16 * wave;
+    f4* s_part = reinterpret_cast<f4*>(s_x + ks * (2 * kUnitBytes + 16));
+    const uint32_t lds0 = __builtin_amdgcn_readfirstlane(lds_address(ring));
 
-    for (int64_t base = (int64_t)blockIdx.x * RPI; base < rows; base += stride) {   // uniform per workgroup
-        const int64_t r = base + wave / KS;
-        float acc[kTok4] = {0.f, 0.f, 0.f, 0.f};
-        if (r < rows) {
-            const uint8_t* wr = w + r * row_bytes;
-            u4 hdr[STEPS];
-            Nib<LPS_> nib[STEPS];
+    // this workgroup's 16-row blocks, one after the other
+    const int bid = (int)blockIdx.x;
+    const int my = share + (bid < extra ? 1 : 0);
+    const int64_t rb0 = (int64_t)bid * share + (bid < extra ? bid : extra);
+    // the next unit to fetch: row block at fw with fleft rows from it on, super-block fsb
+    const uint8_t* fw = w + rb0 * 16 * row_bytes;
+    int64_t fleft = rows - rb0 * 16;
+    int fsb = sb_a;
+    // pieces of the three weight loads: row and offset of the lane's piece; the
+    // third's lanes past the weights take the scales and sums
+    uint32_t voff[3];
+    auto set_rows = [&](int nr) {
 #pragma unroll
-            for (int t = 0; t < STEPS; ++t) {
-                const int sb = sb0 + L::kSbPerStep * t;
-                if (sb < nsb) {
-                    const uint8_t* blk = wr + (int64_t)sb * kBlockBytes;
-                    hdr[t] = *reinterpret_cast<const u4*>(blk);
-                    nib[t] = load_nib<LPS_>(blk, c);
-                }
-            }
-#pragma unroll
-            for (int t = 0; t < STEPS; ++t) {
-                const int sb = sb0 + L::kSbPerStep * t;
-                if (sb < nsb) {
-                    const SbW<LPS_> wv = sb_prep<LPS_>(hdr[t], nib[t], grp);
-#pragma unroll
-                    for (int k = 0; k < kTok4; ++k)
-                        acc[k] += sb_dot<LPS_>(wv, sb * kQK + elo, s_q + k * cols, s_d + k * (cols / 32),
-                                         s_s + k * (cols / 16));
-                }
-            }
+        for (int i = 0; i < 3; ++i) {
+            const int e = lane + 64 * i < 144 ? lane + 64 * i : 143;
+            const int r = e / 9;
+            voff[i] = (uint32_t)(r < nr ? r : nr - 1) * row_bytes + 16u * (e - 9 * r);
         }
-#pragma unroll
-        for (int k = 0; k < kTok4; ++k)
-#pragma unroll
-            for (int o = 32; o > 0; o >>= 1) acc[k] += __shfl_xor(acc[k], o, 64);
-        if constexpr (KS == 1) {
-            if (lane == 0 && r < rows)
-#pragma unroll
-                for (int k = 0; k < kTok4; ++k) out[k * rows + r] = acc[k];
-        } else {
-            if (lane == 0)
-#pragma unroll
-                for (int k = 0; k < kTok4; ++k) s_part[wave][k] = acc[k];
-            __syncthreads();
-            if (part == 0 && lane < kTok4 && r < rows) {
-                float sum = s_part[wave][lane];
-#pragma unroll
-                for (int p = 1; p < KS; ++p) sum += s_part[wave + p][lane];
-                out[lane * rows + r] = sum;
-            }
-            __syncthreads();
+    };
+    set_rows(fleft < 16 ? (int)fleft : 16);
+    const int xe = lane - 16;                  // 0..7: scales, 8..23: sums (the rest as the last)
+    const char* xbase = xe < 8 ? reinterpret_cast<const char*>(xd + (xe >> 1) * (cols / 32)) + 16 * (xe & 1)
+                               : reinterpret_cast<const char*>(xs + (xe < 24 ? (xe - 8) >> 2 : 3) * (cols / 16)) +
+                                     16 * (xe < 24 ? (xe - 8) & 3 : 3);
+    const int xstep = xe < 8 ? 32 : 64;
+    const uint32_t aoff = (lane >> 4) * cols + 16 * (lane & 15);
+    auto fetch = [&](uint32_t buf) {
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");       // the buffer's last reads are done
+        const uint8_t* base = fw + fsb * kBlockBytes;
+        stream_load(base, voff[0], lds0 + buf);
+        stream_load(base, voff[1], lds0 + buf + 1024);
+        const char* p = lane < 16 ? reinterpret_cast<const char*>(base) + voff[2] : xbase + fsb * xstep;
+        stream_load_at(p, lds0 + buf + 2048);
+        stream_load(xq + fsb * kQK, aoff, lds0 + buf + kUnitA);
+        if (++fsb == sb_b) {                   // on to the next row block
+            fsb = sb_a;
+            fw += 16 * row_bytes;
+            fleft -= 16;
+            if (fleft < 16 && fleft > 0) set_rows((int)fleft);
         }
+    };
+    const int n_units = my * (sb_b - sb_a);
+    fetch(0);
+    if (lane == 0) *reinterpret_cast<f4*>(s_zero) = f4{0.f, 0.f, 0.f, 0.f};
+
+    int64_t left = rows - rb0 * 16;
+    float* op = out + rb0 * 16;
+    auto put = [&](int parity, float* o, int64_t n) {             // the sums of a row block of n rows (or more)
+        const int r = tid & 15, tok = tid >> 4;
+        if (tid >= 64 || r >= n) return;
+        const float* p = reinterpret_cast<const float*>(s_part + parity * ks * 16 + r) + tok;
+        float v = *p;
+        for (int u = 1; u < ks; ++u) v += p[64 * u];
+        o[tok * rows + r] = v;
+    };
+    const uint32_t woff = c * kBlockBytes;
+    const uint32_t noff = woff + 16 + 32 * (g >> 1) + 16 * (g & 1);
+    const bool live = (j >> 1) == (g >> 1);
+    const uint32_t coff = kUnitA + t * kQK + 32 * j + 16 * (g & 1);
+    const bool is_d = j == 0;
+    const uint32_t xoff = kUnitX + (is_d ? t * 32 + 4 * g : 128 + t * 64 + 8 * g);
+    const uint32_t xhalf = is_d ? 16 : 32;
+    uint32_t buf = 0;                          // the unit being multiplied
+    int to_come = n_units - 1;                 // units after it
+    f4 acc = {0.f, 0.f, 0.f, 0.f};             // tokens 0..3 of row c, sub-blocks 4h+g
+    for (int b = 0; b < my; ++b) {
+        for (int sb = sb_a; sb < sb_b; ++sb) {
+            if (to_come > 0) {
+                fetch(kUnitBytes - buf);       // into the buffer of the unit before
+                asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kUnitLoads) : "memory");
+            } else {
+                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            }
+            --to_come;
+            const unsigned char* u = ring + buf;
+            const u4 hd = *reinterpret_cast<const u4*>(u + woff);
+            const float dd = half_to_float(hd[0] & 0xFFFFu);
+            const float dm = half_to_float(hd[0] >> 16);
+            const uint32_t b0 = hd[1] >> (8 * g), b1 = hd[2] >> (8 * g), b2 = hd[3] >> (8 * g);
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const u4 raw = *reinterpret_cast<const u4*>(u + noff + 64 * h);
+                const i4 a = *reinterpret_cast<const i4*>(live ? u + coff + 128 * h : s_zero);
+                const int32_t* xp = reinterpret_cast<const int32_t*>(u + xoff + h * xhalf);
+                const int32_t x0 = xp[0], x1 = xp[1];
+                i4 lo, hi;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    lo[e] = (int)(raw[e] & 0x0F0F0F0Fu);
+                    hi[e] = (int)((raw[e] >> 4) & 0x0F0F0F0Fu);
+                }
+                const i4 c0 = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, lo, i4{0, 0, 0, 0}, 0, 0, 0);
+                const i4 c1 = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, hi, i4{0, 0, 0, 0}, 0, 0, 0);
+                // get_scale_min_k4 of sub-block 4h + g
+                const uint32_t sc = h ? (b2 & 0xF) | ((b0 >> 6 & 3) << 4) : b0 & 63;
+                const uint32_t mn = h ? (b2 >> 4 & 0xF) | ((b1 >> 6 & 3) << 4) : b1 & 63;
+                const float al = dd * (float)sc, bl = dm * (float)mn;
+                const float x = __builtin_bit_cast(float, x0), sm = (float)(x0 + x1);   // exact: |sum| <= 32 * 127
+                const float v[4] = {row_lane<4>(sm), row_lane<5>(sm), row_lane<6>(sm), row_lane<7>(sm)};
+                const float dx[4] = {row_lane<0>(x), row_lane<1>(x), row_lane<2>(x), row_lane<3>(x)};
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    acc[i] += dx[i] * (al * (float)(g & 1 ? c1[i] : c0[i]) - bl * v[i]);
+            }
+            buf = kUnitBytes - buf;
+        }
+        // over the four groups of lanes, then with the other waves' after the barrier
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(acc[i]), __float_as_uint(acc[i]), false, false);
+            acc[i] = __uint_as_float(p[0]) + __uint_as_float(p[1]);
+            const auto q = __builtin_amdgcn_permlane32_swap(__float_as_uint(acc[i]), __float_as_uint(acc[i]), false, false);
+            acc[i] = __uint_as_float(q[0]) + __uint_as_float(q[1]);
+        }
+        if (g == 0) s_part[((b & 1) * ks + wave) * 16 + c] = acc;
+        acc = f4{0.f, 0.f, 0.f, 0.f};
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        put(b & 1, op, left);                  // the next write here comes after the next barrier
+        left -= 16;
+        op += 16;
     }
 }
 
@@ -544,129 +664,17 @@ __global__ void __launch_bounds__(QT4) gemv4_kernel(const uint8_t* __restrict__ 
 // tail (measured: gate projection 9.8 -> 9.0 us against a fixed cap of 8
 // workgroups per CU, of which 7 fit).
 template <typename K>
-int gemv_grid(K kernel, int64_t rows, int rows_per_wg, size_t lds, int block = QT) {
+int gemv_grid(K kernel, int64_t rows, int rows_per_wg, size_t lds) {
     int dev = 0, cus = 0, per_cu = 0;
     NOVA_HIP(hipGetDevice(&dev));
     NOVA_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-    NOVA_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, block, lds));
+    NOVA_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, QT, lds));
     if (per_cu < 1) per_cu = 1;
     const int64_t want = (rows + rows_per_wg - 1) / rows_per_wg;
     const int64_t cap = (int64_t)per_cu * cus;
     return (int)(want < cap ? want : cap);
 }
 
-
-// Four tokens on the matrix cores.  v_mfma_i32_16x16x64_i8 multiplies the
-// codes (A: lane (g,r) with r = 4j + t holds token t's 16 codes at positions
-// 16(g&1).. of sub-block 2p + (g>>1) when j is that sub-block's index within
-// its half super-block, zeros otherwise) by 16 weight rows (B: lane (g,c)
-// holds row c's 16 nibble bytes of sub-block pair p at offset 16(g&1), low
-// nibbles for g < 2 and high nibbles for g >= 2: the same positions).  Two
-// MFMAs (pairs 2h, 2h+1) give one C tile of integer dot products whose rows
-// are (sub-block 4h+j, token t) and columns the weight rows, so lane (g,c)
-// holds the four tokens of sub-block 4h+g for row c: one header load and one
-// scale decode serve four values, which the float combination of sb_dot turns
-// into dx * (d*sc*sum(q*c) - dmin*m*sum(c)).  The VALU keeps the nibble
-// unpacking and that epilogue; the dot products move to the matrix core.  ks
-// waves split a 16-row block's super-blocks and add their sums through LDS in
-// a fixed order; 16 / ks blocks per workgroup iteration.
-template <int STEPS>
-__global__ void __launch_bounds__(QT4) gemv4_mfma_kernel(const uint8_t* __restrict__ w, int64_t rows, int cols,
-                                                          const int8_t* __restrict__ xq, const float* __restrict__ xd,
-                                                          const int32_t* __restrict__ xs, float* __restrict__ out,
-                                                          int ks) {
-    extern __shared__ __attribute__((aligned(16))) unsigned char s_x[];
-    __shared__ f4 s_part[QT4 / 64][16];
-    int8_t* s_q = reinterpret_cast<int8_t*>(s_x);                                   // [4][cols]
-    float* s_d = reinterpret_cast<float*>(s_x + kTok4 * cols);                       // [4][cols/32]
-    float* s_s = reinterpret_cast<float*>(s_x + kTok4 * cols + 4 * kTok4 * (cols / 32));   // [4][cols/16]
-    stage_q8<QT4, kTok4 * kMaxCols4>(xq, xd, xs, kTok4 * cols, s_q, s_d, s_s);
-    __syncthreads();
-
-    constexpr int WAVES4 = QT4 / 64;
-    const int rbi = WAVES4 / ks;                   // 16-row blocks per workgroup iteration
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int part = wave % ks, rbl = wave / ks;   // rbl >= rbi: an idle wave
-    const int g = lane >> 4, c = lane & 15;
-    const int t = c & 3, j = c >> 2;               // A role: row (j, t)
-    const int nsb = cols / kQK;
-    const int sb_a = part * nsb / ks, sb_b = (part + 1) * nsb / ks;
-    const int64_t row_bytes = (int64_t)nsb * kBlockBytes;
-    const int64_t n_rb = (rows + 15) / 16;
-    const int sh = 4 * (g >> 1);
-    const int8_t* aq = s_q + t * cols + 16 * g;
-    const int cols32 = cols / 32, cols16 = cols / 16;
-
-    for (int64_t base = (int64_t)blockIdx.x * rbi; base < n_rb; base += (int64_t)gridDim.x * rbi) {   // uniform
-        const int64_t rb = base + rbl;
-        const bool live = rbl < rbi && rb < n_rb;
-        const int64_t r0 = rb * 16;
-        const int64_t rw = live && r0 + c < rows ? r0 + c : rows - 1;
-        const uint8_t* wr = w + rw * row_bytes;
-        f4 acc = {0.f, 0.f, 0.f, 0.f};             // tokens 0..3 of row c, sub-blocks 4h+g
-        if (live) {
-            for (int sb0 = sb_a; sb0 < sb_b; sb0 += STEPS) {
-                u4 raw[STEPS][4], hdr[STEPS];
-#pragma unroll
-                for (int u = 0; u < STEPS; ++u) {
-                    const int sb = sb0 + u < sb_b ? sb0 + u : sb0;
-                    const uint8_t* blk = wr + (int64_t)sb * kBlockBytes;
-                    hdr[u] = *reinterpret_cast<const u4*>(blk);
-#pragma unroll
-                    for (int p = 0; p < 4; ++p) raw[u][p] = *reinterpret_cast<const u4*>(blk + 16 + 32 * p + 16 * (g & 1));
-                }
-#pragma unroll
-                for (int u = 0; u < STEPS; ++u) {
-                    if (sb0 + u >= sb_b) break;
-                    const int sb = sb0 + u;
-                    const uint32_t sw[3] = {hdr[u][1], hdr[u][2], hdr[u][3]};
-                    const float dd = half_to_float(hdr[u][0] & 0xFFFFu);
-                    const float dm = half_to_float(hdr[u][0] >> 16);
-#pragma unroll
-                    for (int h = 0; h < 2; ++h) {
-                        i4 cacc = {0, 0, 0, 0};
-#pragma unroll
-                        for (int q = 0; q < 2; ++q) {
-                            const int p = 2 * h + q;
-                            i4 b;
-#pragma unroll
-                            for (int e = 0; e < 4; ++e) b[e] = (int)((raw[u][p][e] >> sh) & 0x0F0F0F0Fu);
-                            i4 a = {0, 0, 0, 0};
-                            if (j == 2 * q + (g >> 1)) a = *reinterpret_cast<const i4*>(aq + sb * kQK + 64 * p);
-                            cacc = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, b, cacc, 0, 0, 0);
-                        }
-                        const int sub = 4 * h + g;                 // this lane's sub-block
-                        uint32_t sc, mn;
-                        scale_min(sub, sw, sc, mn);
-                        const float al = dd * (float)sc, bl = dm * (float)mn;
-                        const int k0 = sb * kQK + 32 * sub;
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) {
-                            const float dx = s_d[i * cols32 + (k0 >> 5)];
-                            const float sm = s_s[i * cols16 + (k0 >> 4)] + s_s[i * cols16 + (k0 >> 4) + 1];
-                            acc[i] += dx * (al * (float)cacc[i] - bl * sm);
-                        }
-                    }
-                }
-            }
-        }
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            acc[i] += __shfl_xor(acc[i], 16, 64);
-            acc[i] += __shfl_xor(acc[i], 32, 64);
-        }
-        if (g == 0) s_part[wave][c] = acc;
-        __syncthreads();
-        if (part == 0 && g == 0 && live && r0 + c < rows) {
-            f4 sum = s_part[wave][c];
-            for (int pp = 1; pp < ks; ++pp) sum += s_part[wave + pp][c];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) out[(int64_t)i * rows + r0 + c] = sum[i];
-        }
-        __syncthreads();
-    }
-}
 
 template <int STEPS, bool kF32>
 void launch_fixed(const GemvSet& g, size_t lds, hipStream_t s) {
@@ -680,67 +688,44 @@ void launch_split(const GemvSet& g, size_t lds, hipStream_t s) {
     hipLaunchKernelGGL(k, dim3((unsigned)gemv_grid(k, g.end[g.n - 1], 1, lds)), dim3(QT), lds, s, g);
 }
 
-template <int STEPS, int KS>
-void launch_gemv4_shape(const uint8_t* blocks, int64_t rows, int cols, const int8_t* xq, const float* xd,
-                        const int32_t* xs, float* out, size_t lds, hipStream_t s) {
-    auto k = gemv4_kernel<STEPS, KS>;
+// Waves per 16-row block: the fewest rounds of resident workgroups (LDS bounds
+// them) times the units that each of their waves takes, and among equals the
+// fewest waves: more of them only split the sums further.  Within 4% of the best
+// of 1..16 on the shapes above.
+void launch_gemv4(const uint8_t* blocks, int64_t rows, int cols, const int8_t* xq, const float* xd, const int32_t* xs,
+                  float* out, hipStream_t s) {
     static std::once_flag once;                // dynamic LDS beyond 64 KB must be allowed per kernel
     std::call_once(once, [&] {
-        NOVA_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                     (int)(kTok4 * (size_t)kMaxCols4 * 11 / 8)));
+        NOVA_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(gemv4_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, kLdsMax));
     });
-    hipLaunchKernelGGL(k, dim3((unsigned)gemv_grid(k, rows, (QT4 / 64) / KS, lds, QT4)), dim3(QT4), lds, s, blocks,
-                       rows, cols, xq, xd, xs, out);
-}
-
-// Matrices of at least this many weights take the MFMA kernel.  Measured
-// (7B shapes, four tokens): gate 18944 x 3584 18.9 -> 11.7 us, down
-// 3584 x 18944 23.2 -> 15.1 us; the 3584 x 3584 and 512 x 3584 projections
-// stay a little faster on the dot4 kernel (5.9 vs 6.0 us, 5.4 vs 5.65 us):
-// 224 or fewer 16-row blocks are too few to fill the chip's 16-wave
-// workgroups.
-constexpr int64_t kMfma4MinWeights = (int64_t)32 << 20;
-void launch_gemv4_mfma(const uint8_t* blocks, int64_t rows, int cols, const int8_t* xq, const float* xd,
-                       const int32_t* xs, float* out, size_t lds, hipStream_t s) {
-    auto k = gemv4_mfma_kernel<2>;             // 2 super-blocks per load batch (3: gate slower, 4: both)
-    static std::once_flag once;                // dynamic LDS beyond 64 KB must be allowed per kernel
-    std::call_once(once, [&] {
-        NOVA_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                     (int)(kTok4 * (size_t)kMaxCols4 * 11 / 8)));
-    });
-    int dev = 0, cus = 0, per_cu = 0;
+    int dev = 0, cus = 0;
     NOVA_HIP(hipGetDevice(&dev));
     NOVA_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-    NOVA_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k, QT4, lds));
-    if (per_cu < 1) per_cu = 1;
+    auto lds_of = [](int k) { return (size_t)k * (2 * kUnitBytes + 16 + 2 * 16 * 16); };
     const int64_t n_rb = (rows + 15) / 16;
-    const int64_t cap = (int64_t)per_cu * cus;
     const int nsb = cols / kQK;
-    // waves per 16-row block (1..16; 16 / ks blocks per workgroup iteration,
-    // the rest of the 16 waves idle): the fewest rounds of resident
-    // workgroups times super-blocks per wave
     int ks = 1;
     int64_t best = INT64_MAX;
-    for (int kk = 1; kk <= QT4 / 64; ++kk) {
-        const int64_t wgs = (n_rb + (QT4 / 64) / kk - 1) / ((QT4 / 64) / kk);
-        const int64_t cost = (wgs + cap - 1) / cap * ((nsb + kk - 1) / kk);
+    for (int k = 1; k <= kMaxKs4 && k <= nsb && lds_of(k) <= (size_t)kLdsMax; ++k) {
+        const int64_t cap = (int64_t)cus * (kLdsMax / lds_of(k));
+        const int64_t cost = (n_rb + cap - 1) / cap * ((nsb + k - 1) / k);
         if (cost < best) {
             best = cost;
-            ks = kk;
+            ks = k;
         }
     }
-    const int rbi = (QT4 / 64) / ks;
-    const int64_t want = (n_rb + rbi - 1) / rbi;
-    hipLaunchKernelGGL(k, dim3((unsigned)(want < cap ? want : cap)), dim3(QT4), lds, s, blocks, rows, cols, xq, xd, xs,
-                       out, ks);
+    const int64_t cap = (int64_t)cus * (kLdsMax / lds_of(ks));
+    NOVA_REQUIRE(n_rb < (int64_t)1 << 31);
+    const int grid = (int)(n_rb < cap ? n_rb : cap);
+    hipLaunchKernelGGL(gemv4_kernel, dim3(grid), dim3(64 * ks), lds_of(ks), s, blocks, rows, cols, xq, xd, xs, out,
+                       (int)(n_rb / grid), (int)(n_rb % grid));
 }
 
 template <bool kF32>
 void launch_set(const GemvSet& g, hipStream_t st) {
     const int cols = g.cols;
     const size_t lds = (size_t)cols + 4 * (size_t)(cols / 32) + 4 * (size_t)(cols / 16);
-    constexpr int SPS = Lanes<kLps1>::kSbPerStep;
-    switch ((cols / kQK + SPS - 1) / SPS) {    // steps of SPS super-blocks
+    switch ((cols / kQK + kSbPerStep - 1) / kSbPerStep) {
         case 1: launch_fixed<1, kF32>(g, lds, st); break;
         case 2: launch_fixed<2, kF32>(g, lds, st); break;
         case 3: launch_fixed<3, kF32>(g, lds, st); break;
@@ -794,25 +779,7 @@ void launch_gemv4_q4k(const uint8_t* blocks, int64_t rows, int cols, const int8_
     NOVA_REQUIRE(cols > 0 && cols % kQK == 0 && cols <= kMaxCols4);
     NOVA_REQUIRE(aligned16(xq) && aligned16(xd) && aligned16(xs));   // staged with 16 B loads
     if (rows == 0) return;
-    const size_t lds = kTok4 * ((size_t)cols + 4 * (size_t)(cols / 32) + 4 * (size_t)(cols / 16));
-    const hipStream_t st = reinterpret_cast<hipStream_t>(s);
-    if (rows * (int64_t)cols >= kMfma4MinWeights) {
-        launch_gemv4_mfma(blocks, rows, cols, xq, xd, xs, out, lds, st);
-        NOVA_LAUNCHED();
-        return;
-    }
-    constexpr int SPS = Lanes<kLps4>::kSbPerStep;
-    switch ((cols / kQK + SPS - 1) / SPS) {    // steps of SPS super-blocks: the row shapes
-        case 1: launch_gemv4_shape<1, 1>(blocks, rows, cols, xq, xd, xs, out, lds, st); break;
-        case 2: launch_gemv4_shape<2, 1>(blocks, rows, cols, xq, xd, xs, out, lds, st); break;
-        case 3: launch_gemv4_shape<3, 1>(blocks, rows, cols, xq, xd, xs, out, lds, st); break;
-        case 4: launch_gemv4_shape<4, 1>(blocks, rows, cols, xq, xd, xs, out, lds, st); break;
-        case 5: case 6: case 7: case 8: launch_gemv4_shape<2, 4>(blocks, rows, cols, xq, xd, xs, out, lds, st); break;
-        case 9: case 10: case 11: case 12:
-            launch_gemv4_shape<3, 4>(blocks, rows, cols, xq, xd, xs, out, lds, st);
-            break;
-        default: launch_gemv4_shape<4, 4>(blocks, rows, cols, xq, xd, xs, out, lds, st); break;
-    }
+    launch_gemv4(blocks, rows, cols, xq, xd, xs, out, reinterpret_cast<hipStream_t>(s));
     NOVA_LAUNCHED();
 }
 

@@ -170,3 +170,11 @@ def test_gemv4_matches_single_token(rows, cols, nova7, oracle):
         assert np.all(err <= 2e-6 * scale), f"token {t}: max err/scale {np.max(err / scale):.2e}"
         diff = np.abs(got[t][check].astype(np.float64) - one[check])
         assert np.all(diff <= 4e-6 * scale), f"token {t} vs one-token: {np.max(diff / scale):.2e}"
+
+
+@pytest.mark.parametrize("rows,cols", [(1, 256), (15, 512), (17, 768), (40, 28672), (9301, 1024), (74003, 256)])
+def test_gemv4_edges(rows, cols, nova7, oracle):
+    """One super-block per row (one wave per 16-row block), ragged last blocks,
+    the widest rows, and more blocks than fit at once (a workgroup walks several,
+    its last one ragged)."""
+    test_gemv4_matches_single_token(rows, cols, nova7, oracle)
