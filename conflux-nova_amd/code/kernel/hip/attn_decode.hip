@@ -21,13 +21,19 @@
 //    the bytes it saves).  The reference-signature path writes one partial per
 //    head and page range (its scratch holds 32 rows per head; there each page
 //    range runs as NKV workgroups, one per kv head, so one single-session call
-//    spreads over 31 * NKV CUs).
-//    Every wave derives the partition itself from one load of n_keys.
+//    spreads over 31 * NKV CUs).  The batched partition is worked out on the
+//    device once per step (the plan), the one-session call's on the host.
 //  * One workgroup = 8 wave64s, one workgroup per CU.  Wave w serves kv head
 //    w % NKV and takes every R-th pair of pages (R = 8/NKV), so the workgroup
 //    reads whole 16-token pages (all kv heads) and each wave streams 256 B rows
-//    of its head; the CU keeps 8 pairs (128 KiB) of K/V outstanding.  The
-//    query operands live once per kv head in LDS.
+//    of its head; the CU keeps 8 pairs (128 KiB) of K/V outstanding.
+//  * Loads in address order.  The vector L1 takes one 128 B line of an
+//    instruction per clock, so a 16 B/lane load whose 64 lanes lie on 16 rows
+//    costs it four times one whose lanes follow each other.  Query rows are
+//    therefore read lane by lane along the row and K as whole 256 B rows, and
+//    both change into the MFMA's operand order in LDS (K 16 B chunk k of row r
+//    at position k ^ r: no bank conflicts either way).  28 layers of 24 solo
+//    sessions of 17 to 512 keys, 7B shapes: 377 us with operand-order loads, 349.
 //  * Latency hiding inside a wave: the segment's block-table slice is fetched
 //    once (one coalesced load, then v_readlane per page), so no pair waits on
 //    a table lookup.  Every wave issues its loads in one fixed order -- the
@@ -47,10 +53,12 @@
 //    and the V operand is read as 16 B per lane straight from 256 B rows.
 //  * fp32-grade accuracy from fp16 operands.  K and V are fp16 in the pool (exact
 //    MFMA inputs).  Q (fp32) is split q = hi + lo into two fp16 terms after a
-//    per-head power-of-two scaling, P (fp32 softmax weights) likewise; each
-//    product is two MFMAs accumulating in fp32, leaving ~2^-22 relative error
-//    per operand instead of fp16's 2^-11.  The matrix cores have the slack:
-//    the kernel is bound by HBM, not by MFMA issue.
+//    per-head power-of-two scaling, P (fp32 softmax weights) likewise, leaving
+//    ~2^-22 relative error per operand instead of fp16's 2^-11.  A GQA group has
+//    at most 8 heads and the MFMA 16 columns: columns 0..7 take the hi terms,
+//    8..15 the lo terms of the same heads, so each product is one MFMA and one
+//    conversion in the registers of each wave, both terms accumulating in fp32.  Scores add their two
+//    columns once per pair (a DPP move within the row), O once per workgroup.
 //  * Online softmax in the log2 domain (raw v_exp_f32), scale*log2(e) folded
 //    into the per-head factor, with a lazy running max: it moves only when a
 //    score exceeds it by more than 8, so most pairs skip the cross-lane max
@@ -89,6 +97,7 @@ constexpr int NH = Model::NH, NKV = Model::NKV, HD = Model::HD, G = Model::G, KV
 #endif
 constexpr int WAVES = NOVA_DECODE_WAVES;
 constexpr int THREADS = WAVES * 64;
+static_assert(G <= 8, "hi and lo terms of a GQA group share the 16 MFMA columns");
 constexpr int R = WAVES / NKV;           // waves per kv head
 static_assert(WAVES % NKV == 0, "kv heads must divide the waves of a workgroup");
 constexpr int PW = HD + 2;               // partial row of the reference-signature scratch: m, l, acc[HD]
@@ -101,6 +110,7 @@ constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLazy = 8.0f;            // running-max slack, log2 units (weights <= 2^8)
 constexpr int64_t kPageBytes = (int64_t)kKvBlock * KVW * 2;
 constexpr int kRowBytes = KVW * 2;
+constexpr int kQStride = HD + 4;                 // floats per query row in LDS (rows on different banks)
 
 struct DecodeArgs {
     const float* q;          // [n_sess][NH][HD]
@@ -120,10 +130,11 @@ struct DecodeArgs {
     const float* cs;         // RoPE table rows [pos][HD/2] (null: no rotation)
     const float* sn;
     float* part;             // [(Gw + n_sess) * (wave_parts ? R : 1)][NH][PW]
-    const int32_t* plan;     // per-step plan (null: derive the partition in-kernel)
+    const int32_t* plan;     // per-step plan (null: kv-split and solo launches)
     int gw;                  // workgroups in the grid
     int wave_parts;          // 1: a partial slot per (workgroup, wave row), no in-workgroup merge
     int kv_split;            // 1: grid.x = kv head, all waves of a workgroup on that head
+    int n_pages, n_ranges;   // kv-split launches of one session: its pages and page ranges (grid.y)
     float* o;                // solo launches: the output [n_sess][NH][HD], written by the split kernel
     int tab_read;            // solo launches: block-table entries of a row that may be read before n_keys is known
     int spin;                // polls of the in-workgroup exchange before it gives up (kSpinLimit)
@@ -179,26 +190,29 @@ __host__ __device__ constexpr int64_t plan_status_off(int n_sess, int gw) {
 __host__ __device__ constexpr int64_t plan_ints(int n_sess, int gw) { return plan_status_off(n_sess, gw) + 1; }
 
 __device__ __forceinline__ float shfl_xor_f(float v, int m) { return __shfl_xor(v, m, 64); }
+// lane c ^ 8 of each row of 16 lanes (row_ror:8)
+__device__ __forceinline__ float swap_halves(float v) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x128, 0xF, 0xF, true));
+}
 
 // K/V page loads go out non-temporal: each byte is read once per launch, and
-// every load instruction covers whole 128 B lines (V: 256 B row slices; K:
-// 8 rows x 128 B, see k_operand).  Measured: page-sized non-temporal
-// streaming reaches 6.9 TB/s against 6.1 TB/s with the default policy; V
-// non-temporal took the config-2 step 0.905 -> 0.875 ms, K with whole-line
-// loads 0.834-0.841 -> 0.826 ms (config 4: 6.21 -> 6.37-6.55 TB/s).  K
+// every load instruction covers whole 256 B row slices (K: rows 4i + g, V:
+// rows 4g + j of the 16 lanes g).  Measured: page-sized non-temporal
+// streaming reaches 6.9 TB/s against 6.1 TB/s with the default policy.  K
 // loaded the MFMA's way (64 B of 16 rows per instruction, the other half of
-// each line by the next one) is slower non-temporal: 0.97 ms.
+// each line by the next one) is slower non-temporal: 0.97 against 0.83 ms per
+// config-2 step.
 // Each page is a buffer resource: the loads take the page base in SGPRs and a
-// 32-bit lane offset with an immediate, instead of a 64-bit VGPR address per
-// load (the double-buffered solo loop: 254 -> 217 VGPRs, and its prefetch no
-// longer waits on address registers still being loaded).  num_records bounds
+// 32-bit lane offset with a scalar one, instead of a 64-bit VGPR address per
+// load (and the solo loop's prefetch does not wait on address registers still
+// being loaded).  num_records bounds
 // every load to its page; num_records = 0 makes a load return zero without a
 // memory access (a prefetch slot with no pair left).
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t page_rsrc(const char* base, int bytes) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(base), 0, bytes, 0x00020000);
 }
-__device__ __forceinline__ u4 ldb16_nt(__amdgpu_buffer_rsrc_t r, uint32_t off) {
-    return __builtin_bit_cast(u4, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 2));   // aux 2: nt
+__device__ __forceinline__ u4 ldb16_nt(__amdgpu_buffer_rsrc_t r, uint32_t off, uint32_t soff = 0) {
+    return __builtin_bit_cast(u4, __builtin_amdgcn_raw_buffer_load_b128(r, off, soff, 2));   // aux 2: nt
 }
 
 // Pages per workgroup: the even share ceil(T / gw), but at least kMinShare so
@@ -213,16 +227,21 @@ __host__ __device__ __forceinline__ int share_of(int T, int gw) {
 }
 
 // Page range of workgroup j of a session with `pages` pages split over k
-// workgroups: [j*pages/k, (j+1)*pages/k).  The plan kernel, the in-kernel
-// partition and the combine's row count all take it from here, so a range
+// workgroups: [j*pages/k, (j+1)*pages/k).  The plan kernel, the kv-split
+// launch and the combine's row count all take it from here, so a range
 // never exceeds range_max_pages(pages, k).
 __host__ __device__ __forceinline__ int range_begin(int j, int pages, int k) {
     return (int)((int64_t)j * pages / k);
 }
+// the same in 32 bits, for the few ranges of a kv-split launch (j <= 31, and
+// an int's worth of keys is at most 2^27 pages)
+__device__ __forceinline__ int range_begin32(int j, int pages, int k) {
+    return (int)((uint32_t)j * (uint32_t)pages / (uint32_t)k);
+}
 __host__ __device__ __forceinline__ int range_max_pages(int pages, int k) { return (pages + k - 1) / k; }
 
-// The batch partition, derived by one wave from n_keys (every wave that needs
-// it computes it; no LDS, no barrier).  P_i = pages of session i, T = sum P_i,
+// The batch partition, derived by one wave of the plan kernel from n_keys (no
+// LDS, no barrier).  P_i = pages of session i, T = sum P_i,
 // target = max(ceil(T / gw), 4), k_i = ceil(P_i / target) workgroups for session i,
 // kc_i = k_0 + ... + k_{i-1} its first workgroup (= its first partial slot).
 // Sum k_i <= gw + n_sess, so the grid launches gw + n_sess workgroups.
@@ -264,9 +283,8 @@ __device__ int plan_share(const DecodeArgs& a, int T) {
     return target;
 }
 
-// Find the session that owns workgroup slot w (find_slot) or the partition
-// entry of session `want` (want >= 0).
-__device__ Part partition(const DecodeArgs& a, int w, int want) {
+// The session that owns workgroup w of the batch and its partition entry.
+__device__ Part partition(const DecodeArgs& a, int w) {
     const int lane = threadIdx.x & 63;
     int T = 0;
     for (int base = 0; base < a.n_sess; base += 64) {
@@ -293,7 +311,7 @@ __device__ Part partition(const DecodeArgs& a, int w, int want) {
             if (lane >= o) incl += t;
         }
         const int kc = carry + incl - k;
-        const bool hit = want >= 0 ? (i == want) : (i < a.n_sess && k > 0 && kc <= w && w < kc + k);
+        const bool hit = i < a.n_sess && k > 0 && kc <= w && w < kc + k;
         const uint64_t b = __builtin_amdgcn_ballot_w64(hit);
         if (b) {
             const int src = __builtin_ctzll(b);
@@ -338,29 +356,9 @@ __device__ int sum_k(const DecodeArgs& a) {
 
 // K and V operands of one pair of pages, as loaded
 struct PairRegs {
-    u4 k0[4], k1[4];   // K of page 0 / page 1 as whole-line loads (k_operand)
+    u4 k0[4], k1[4];   // K of page 0 / page 1: lane (g,c) of k[i] has row 4i + g, halfs [8c, +8)
     u4 v[8];           // V rows kappa(g,j) = (page j/4, slot 4g + j%4), halves [8c, +8)
 };
-
-// K operand ks of one page from the whole-line loads.  Load 2h+0 (X) holds,
-// in lane (g,c), row c&7 at bytes 128h + 16(g + 4(c>>3)); load 2h+1 (Y) the
-// same for rows 8 + (c&7).  The MFMA wants row c at bytes 64ks + 16g: for
-// even ks that is X in lanes c < 8 and Y of lane c-8 in lanes c >= 8; for odd
-// ks, X of lane c+8 in lanes c < 8 and Y in lanes c >= 8.  A row_ror:8 DPP
-// move writing only the banks (4-lane groups) of the lanes that need it
-// builds each operand dword in one instruction.
-__device__ __forceinline__ u4 k_operand(const u4* kl, int ks) {
-    const u4 x = kl[ks & 2], y = kl[(ks & 2) + 1];
-    u4 r;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        if (ks & 1)
-            r[e] = (uint32_t)__builtin_amdgcn_update_dpp((int)y[e], (int)x[e], 0x128, 0xF, 0x3, false);
-        else
-            r[e] = (uint32_t)__builtin_amdgcn_update_dpp((int)x[e], (int)y[e], 0x128, 0xF, 0xC, false);
-    }
-    return r;
-}
 
 // kSolo (with kKvSplit): one workgroup per (kv head, session) streams all of
 // the session's pages for that head, merges its waves in LDS and writes the
@@ -375,23 +373,29 @@ __global__ void __launch_bounds__(THREADS)
 decode_split_kernel(DecodeArgs a) {
     static_assert(!kSolo || kKvSplit, "solo workgroups serve one kv head");
     static_assert(!kSingle || !kKvSplit, "single-session launches use the planned grid");
-    // two page pairs in flight per wave (the next pair's loads go out before
-    // this pair's arithmetic): solo workgroups only.  The split grid is
-    // slower with it even at 242 VGPRs with no spills and the prefetch in
-    // flight (config 2 split kernel 26.5-27.0 vs 23.6-24.6 us, config 1
-    // 8.0 vs 6.15 us, config 4 unchanged): its 8 waves per CU already keep
-    // enough of the chip's bytes in flight.
+    // Pairs in flight.  Solo workgroups: two per wave (the next pair's loads go
+    // out before this pair's arithmetic).  The planned grid of several sessions
+    // with two or more waves per kv head: half a pair more (kAhead, below); a
+    // whole one is slower there (config-2 split kernel 26.5-27.0 against
+    // 23.6-24.6 us).  Everything else: one pair, the 8 waves of the CU overlap
+    // each other's latency.
     constexpr bool kDB = kSolo;
+    constexpr bool kAhead = R > 1 && !kKvSplit && !kSingle;
     __shared__ float s_m[WAVES][16];
     __shared__ float s_l[WAVES][16];
     __shared__ float s_acc[(R > 1 || kKvSplit) ? WAVES : 1][G][HD];
-    __shared__ u4 s_q[NKV][4][2][64];            // Q^T hi/lo operands per kv head
-    __shared__ float s_qf[NKV][16];              // per-head score factor
+    constexpr int kQRows = kKvSplit ? G : NH;    // query rows this workgroup serves
+    __shared__ __attribute__((aligned(16))) float s_q[kQRows][kQStride];   // as given (fp32)
+    __shared__ u4 s_k[WAVES][2][256];            // each wave's pair of K pages, on its way into operand order
     __shared__ int s_ready[WAVES];               // a wave's exchange rows are in LDS (one-slot partials)
 
     const int tid = threadIdx.x;
-    // solo: the wave index (and the pair loop) kept in scalar registers
-    const int wave = kDB ? __builtin_amdgcn_readfirstlane(tid >> 6) : tid >> 6;
+    // the wave index, and with it the pair loop and the page resources, in scalar
+    // registers; not in a single session's step, whose waves take about one pair
+    // each and have nothing to gain from it (28 1.5B layers of
+    // 1040 keys: 274 us against 279 with it and 286 before K went through LDS)
+    constexpr bool kUniform = !kSingle;
+    const int wave = kUniform ? __builtin_amdgcn_readfirstlane(tid >> 6) : tid >> 6;
     const int lane = tid & 63;
     const int g = lane >> 4;      // 0..3
     const int c = lane & 15;      // 0..15
@@ -416,9 +420,11 @@ decode_split_kernel(DecodeArgs a) {
     constexpr int kAppW = kKvSplit ? HD : KVW;      // halfs of the row this workgroup appends
     const int app_off = kKvSplit ? kvh * HD : 0;
     const bool app_lane = !kRope && tid < kAppW / 8;
-    const bool qreal = c < G;
+    const int qc = c & 7;         // the head of MFMA columns c and c ^ 8
+    const bool qreal = qc < G;
     u4 knew, vnew;
-    f4 qraw[8];
+    constexpr int kQUnits = kQRows * HD / 4, kQLoads = (kQUnits + THREADS - 1) / THREADS;
+    f4 qraw[kQLoads];
     auto issue_new = [&](int sess) {
         const uint16_t* ks = a.k_new ? a.k_new : reinterpret_cast<const uint16_t*>(a.q);
         const uint16_t* vs = a.v_new ? a.v_new : reinterpret_cast<const uint16_t*>(a.q);
@@ -427,14 +433,12 @@ decode_split_kernel(DecodeArgs a) {
         vnew = *reinterpret_cast<const u4*>(vs + src);
     };
     auto issue_q = [&](int sess) {
-        // the converting wave of each kv head (r == 0) reads its rows; the others one line
-        const int64_t qoff = r == 0 ? ((int64_t)sess * NH + kvh * G + (qreal ? c : 0)) * HD + 8 * g : (int64_t)sess * NH * HD;
-        const int step = r == 0 ? 1 : 0;
-        const float* qp = a.q + qoff;
+        // the workgroup's query rows, 16 B per thread and load in address order
+        const float* qp = a.q + ((int64_t)sess * NH + (kKvSplit ? kvh * G : 0)) * HD;
 #pragma unroll
-        for (int ks = 0; ks < 4; ++ks) {
-            qraw[2 * ks] = *reinterpret_cast<const f4*>(qp + step * (32 * ks));
-            qraw[2 * ks + 1] = *reinterpret_cast<const f4*>(qp + step * (32 * ks + 4));
+        for (int e = 0; e < kQLoads; ++e) {
+            const int u = tid + e * THREADS;
+            qraw[e] = *reinterpret_cast<const f4*>(qp + 4 * (u < kQUnits ? u : 0));
         }
     };
     if constexpr (kSolo) {
@@ -444,6 +448,8 @@ decode_split_kernel(DecodeArgs a) {
         const int32_t* trow = a.tables + (int64_t)i * a.table_stride;
         tv = lane < a.tab_read ? trow[lane] : 0;
         tv2 = 64 + lane < a.tab_read ? trow[64 + lane] : 0;
+        issue_new(i);
+        issue_q(i);
         n_keys = nkeys_of(a, i);
         pa = 0;
         pb = n_keys > 0 ? (n_keys + kKvBlock - 1) >> kKvBlockShift : 0;
@@ -452,7 +458,16 @@ decode_split_kernel(DecodeArgs a) {
             for (int e = tid; e < G * HD / 4; e += THREADS) reinterpret_cast<f4*>(orow)[e] = f4{0.f, 0.f, 0.f, 0.f};
             return;
         }
-    } else if (a.plan) {
+    } else if constexpr (kKvSplit) {
+        // page range w of the one session, whose partition the host worked out
+        i = 0;
+        n_keys = a.n_keys_scalar;
+        pa = range_begin32(w, a.n_pages, a.n_ranges);
+        pb = range_begin32(w + 1, a.n_pages, a.n_ranges);
+        tv = pa + lane < pb ? a.tables[pa + lane] : 0;
+        issue_new(0);
+        issue_q(0);
+    } else {
         // one load: lane t holds phys[t]; lanes 0..3 the header
         const int32_t* rec = a.plan + plan_rec_off(a.n_sess) + (int64_t)w * kRec;
         tv = rec[lane];
@@ -471,45 +486,40 @@ decode_split_kernel(DecodeArgs a) {
         pb = __builtin_amdgcn_readlane(hv, 2);
         n_keys = __builtin_amdgcn_readlane(hv, 3);
         slot = __builtin_amdgcn_readlane(hv, 4);
-    } else {
-        const Part pt = partition(a, w, -1);
-        if (pt.sess < 0) return;                 // idle workgroup (uniform)
-        i = pt.sess;
-        n_keys = pt.n_keys;
-        const int j = w - pt.kc;                 // this workgroup's share of session i
-        pa = range_begin(j, pt.pages, pt.k);
-        pb = range_begin(j + 1, pt.pages, pt.k);
-        tv = (pa + lane < pb) ? a.tables[(int64_t)i * a.table_stride + pa + lane] : 0;
     }
-    // settle the slice register here (one wait, nothing else in flight yet):
-    // otherwise the compiler's wait before its first read, after the query and
-    // first-pair loads below are issued, would be a wait for all of them
-    asm volatile("v_mov_b32 %0, %1" : "=v"(tv) : "v"(tv));
-    if constexpr (kSolo) asm volatile("v_mov_b32 %0, %1" : "=v"(tv2) : "v"(tv2));
+    // settle the slice register here (one wait, at most the query and token rows
+    // behind it in flight): otherwise the compiler's wait before its first read,
+    // after the first-pair loads below are issued, would be a wait for all of them
+    if constexpr (kKvSplit) asm volatile("v_mov_b32 %0, %1" : "=v"(tv) : "v"(tv) : "memory");
+    else asm volatile("v_mov_b32 %0, %1" : "=v"(tv) : "v"(tv));
+    if constexpr (kSolo) asm volatile("v_mov_b32 %0, %1" : "=v"(tv2) : "v"(tv2) : "memory");
     const int last_page = (n_keys - 1) >> kKvBlockShift;
     const int32_t* table = a.tables + (int64_t)i * a.table_stride;
 
     // lane-constant byte offsets inside a page
-    const uint32_t koff = (uint32_t)((c & 7) * kRowBytes + kvh * HD * 2 + 16 * (g + 4 * (c >> 3)));
-    uint32_t voff[4];
-#pragma unroll
-    for (int jj = 0; jj < 4; ++jj) voff[jj] = (uint32_t)((4 * g + jj) * kRowBytes + kvh * HD * 2 + 16 * c);
+    const uint32_t koff = (uint32_t)(g * kRowBytes + kvh * HD * 2 + 16 * c);          // K rows 4i + g
+    const uint32_t voff = (uint32_t)(4 * g * kRowBytes + kvh * HD * 2 + 16 * c);      // V rows 4g + j
+    // K in LDS: 16 B chunk k of row r at position k ^ r of the row (free of bank
+    // conflicts both ways): written as loaded, read as the MFMA wants it (row c,
+    // chunk 4ks + g)
+    unsigned char* kt = reinterpret_cast<unsigned char*>(&s_k[wave][0][0]);
+    const uint32_t kwr = (uint32_t)(g * 256 + ((c ^ g) << 4));          // row 4i + g: ^ (i << 6), + 1024 i
+    const uint32_t krd = (uint32_t)(c * 256 + ((g ^ c) << 4));          // chunk 4ks + g: ^ (ks << 6)
 
     const char* pk = reinterpret_cast<const char*>(a.pool_k);
     const char* pv = reinterpret_cast<const char*>(a.pool_v);
     const int64_t layer_page0 = (int64_t)a.layer * a.nb;
 
     {
-        // block-table slice of this workgroup: lane t holds table[pa + 64*chunk + t]
+        // block-table slice of this workgroup: the first 64 (solo: 128) entries
+        // sit in tv (, tv2); later pages come one at a time through the scalar
+        // cache.  No vector load in the pair loop but the pairs', so the
+        // compiler's waits count exactly and what is in flight stays in flight
+        // during the arithmetic.
         int tchunk = 0;
         auto phys_of = [&](int pg) -> int {
             const int rel = pg - pa;
-            if constexpr (kDB) {
-                // the first 64 (solo: 128) entries sit in tv (, tv2); later
-                // pages come one at a time through the scalar cache.  No vector
-                // load in the pair loop but the pairs', so the compiler's waits
-                // count exactly and the prefetched pair stays in flight during
-                // the arithmetic.
+            if constexpr (kUniform) {
                 if (rel < 64) return __builtin_amdgcn_readlane(tv, rel);
                 if (kSolo && rel < 128) return __builtin_amdgcn_readlane(tv2, rel - 64);
                 return *(const __attribute__((address_space(4))) int32_t*)(uintptr_t)(table + pg);
@@ -524,34 +534,43 @@ decode_split_kernel(DecodeArgs a) {
 
         const int npairs = (pb - pa + 1) >> 1;
         // kFirst: a wave's first pair (pages < 16 into the range) takes its pages
-        // straight from the slice register, with no reload branch: a reload's
-        // load would make the first pair's issue wait for every load before it
+        // straight from the slice register, with no branch
         // live == false: the same 16 loads with an empty resource (they
         // return zero, no memory access), for a prefetch slot with no pair
         // left -- a load under a branch would make the compiler drain every
         // load in flight before the next use of any of them
-        auto load_pair = [&](auto first_tag, int qp, PairRegs& pr, bool live = true) {
+        struct PagePair { int ph0, ph1; };
+        auto pages_of = [&](auto first_tag, int qp) -> PagePair {
             constexpr bool kFirst = decltype(first_tag)::value;
             const int pg0 = pa + 2 * qp;
             const int pg1 = pg0 + 1 < pb ? pg0 + 1 : pg0;   // a lone last page loads itself twice
-            const int ph0 = kFirst ? __builtin_amdgcn_readlane(tv, pg0 - pa) : phys_of(pg0);
-            const int ph1 = kFirst ? __builtin_amdgcn_readlane(tv, pg1 - pa) : phys_of(pg1);
-            const int64_t b0 = (layer_page0 + ph0) * kPageBytes;
-            const int64_t b1 = (layer_page0 + ph1) * kPageBytes;
+            return PagePair{kFirst ? __builtin_amdgcn_readlane(tv, pg0 - pa) : phys_of(pg0),
+                            kFirst ? __builtin_amdgcn_readlane(tv, pg1 - pa) : phys_of(pg1)};
+        };
+        auto load_k = [&](const PagePair& pp, PairRegs& pr, bool live = true) {
             const int nr = live ? (int)kPageBytes : 0;
-            const auto rk0 = page_rsrc(pk + b0, nr), rk1 = page_rsrc(pk + b1, nr);
-            const auto rv0 = page_rsrc(pv + b0, nr), rv1 = page_rsrc(pv + b1, nr);
+            const auto r0 = page_rsrc(pk + (layer_page0 + pp.ph0) * kPageBytes, nr);
+            const auto r1 = page_rsrc(pk + (layer_page0 + pp.ph1) * kPageBytes, nr);
 #pragma unroll
-            for (int ks = 0; ks < 4; ++ks) {
-                const uint32_t o = koff + (ks & 1) * 8 * kRowBytes + (ks >> 1) * 128;
-                pr.k0[ks] = ldb16_nt(rk0, o);
-                pr.k1[ks] = ldb16_nt(rk1, o);
+            for (int i4 = 0; i4 < 4; ++i4) {
+                pr.k0[i4] = ldb16_nt(r0, koff, 4 * i4 * kRowBytes);
+                pr.k1[i4] = ldb16_nt(r1, koff, 4 * i4 * kRowBytes);
             }
+        };
+        auto load_v = [&](const PagePair& pp, PairRegs& pr, bool live = true) {
+            const int nr = live ? (int)kPageBytes : 0;
+            const auto r0 = page_rsrc(pv + (layer_page0 + pp.ph0) * kPageBytes, nr);
+            const auto r1 = page_rsrc(pv + (layer_page0 + pp.ph1) * kPageBytes, nr);
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                pr.v[j] = ldb16_nt(rv0, voff[j]);
-                pr.v[4 + j] = ldb16_nt(rv1, voff[j]);
+                pr.v[j] = ldb16_nt(r0, voff, j * kRowBytes);
+                pr.v[4 + j] = ldb16_nt(r1, voff, j * kRowBytes);
             }
+        };
+        auto load_pair = [&](auto first_tag, int qp, PairRegs& pr, bool live = true) {
+            const PagePair pp = pages_of(first_tag, qp);
+            load_k(pp, pr, live);
+            load_v(pp, pr, live);
         };
 
         // Issue order: the appended token's row and the query rows first, then
@@ -565,7 +584,7 @@ decode_split_kernel(DecodeArgs a) {
         const int phys_last = table[last_page];     // the appended token's page (may lie past the slice register)
         static_assert(KVW / 8 <= THREADS, "one 16-byte piece of the appended row per thread");
         const bool app_thread = app_lane && appends;
-        if constexpr (!kSingle) {
+        if constexpr (!kSingle && !kKvSplit) {
             issue_new(i);
             issue_q(i);
         }
@@ -631,18 +650,30 @@ decode_split_kernel(DecodeArgs a) {
             }
         }
 
-        // ---- the query group of each kv head as split fp16 B operands, in LDS ----
-        // lane (g,c): head kvh*G + c, dims d = 32*ks + 8*g + j.  The first wave of
-        // each kv head converts; the R waves of that head read them per pair.
-        if (r == 0) {
+        // ---- the query group of the wave's kv head as split fp16 B operands ----
+        // The rows go through LDS as they are; every wave then takes its operands:
+        // lane (g,c) head kvh*G + (c & 7), dims d = 32*ks + 8*g + j, its hi term for
+        // c < 8 and its lo term otherwise (16 registers).
+#pragma unroll
+        for (int e = 0; e < kQLoads; ++e) {
+            const int u = tid + e * THREADS;
+            if (u < kQUnits) *reinterpret_cast<f4*>(&s_q[u / (HD / 4)][4 * (u % (HD / 4))]) = qraw[e];
+        }
+        if (lane == 0) s_ready[wave] = 0;
+        __syncthreads();                       // also the appended row, before any wave reads its page
+        h8 q8[4];
+        float qf;
+        {
+            const float* qrow = &s_q[(kKvSplit ? 0 : kvh * G) + (qreal ? qc : 0)][8 * g];
             float qv[4][8];
             float amax = 0.f;
 #pragma unroll
             for (int ks = 0; ks < 4; ++ks) {
+                const f4 q0 = *reinterpret_cast<const f4*>(qrow + 32 * ks), q1 = *reinterpret_cast<const f4*>(qrow + 32 * ks + 4);
 #pragma unroll
                 for (int jj = 0; jj < 4; ++jj) {
-                    qv[ks][jj] = qreal ? qraw[2 * ks][jj] : 0.f;
-                    qv[ks][4 + jj] = qreal ? qraw[2 * ks + 1][jj] : 0.f;
+                    qv[ks][jj] = qreal ? q0[jj] : 0.f;
+                    qv[ks][4 + jj] = qreal ? q1[jj] : 0.f;
                 }
             }
             if constexpr (kRope) {
@@ -672,54 +703,52 @@ decode_split_kernel(DecodeArgs a) {
             if (amax > 0.f) (void)frexpf(amax, &ex);
             const int k2 = amax > 0.f ? 15 - ex : 0;    // amax * 2^k2 in [2^14, 2^15)
             const float up = ldexpf(1.f, k2);
-            if (g == 0) s_qf[kvh][c] = kScale * kLog2e * ldexpf(1.f, -k2);
+            qf = kScale * kLog2e * ldexpf(1.f, -k2);
 #pragma unroll
             for (int ks = 0; ks < 4; ++ks) {
-                h8 hi, lo;
 #pragma unroll
                 for (int jj = 0; jj < 8; ++jj) {
                     const float x = qv[ks][jj] * up;
                     const _Float16 h = (_Float16)x;
-                    hi[jj] = h;
-                    lo[jj] = (_Float16)(x - (float)h);
+                    q8[ks][jj] = c < 8 ? h : (_Float16)(x - (float)h);
                 }
-                s_q[kvh][ks][0][lane] = __builtin_bit_cast(u4, hi);
-                s_q[kvh][ks][1][lane] = __builtin_bit_cast(u4, lo);
             }
         }
-        if (lane == 0) s_ready[wave] = 0;
-        __syncthreads();
-        const float qf = s_qf[kvh][c];
+        const float lo_col = c < 8 ? 0.f : 1.f;
 
         float m = -INFINITY, lsum = 0.f;
         f4 acc[8];
 #pragma unroll
         for (int cb = 0; cb < 8; ++cb) acc[cb] = f4{0.f, 0.f, 0.f, 0.f};
 
-        auto compute_pair = [&](int qp, PairRegs& cur) {
+        auto compute_pair = [&](int qp, PairRegs& cur, auto&& k_free) {
             const int pg0 = pa + 2 * qp;
             const bool two = pg0 + 1 < pb;
             // keys that exist: all of them except in the session's last pair
             const bool tail = !two || (((pg0 + 2) << kKvBlockShift) > n_keys);
 
-            // S = K . Q^T  (C layout: lane (g,c) holds keys 4g+i of head c)
-            // hi and lo products in separate accumulators: four chains of four
-            // dependent MFMAs instead of two of eight
+            // S = K . Q^T  (C layout: lane (g,c) holds keys 4g+i of column c: the
+            // hi product of head c for c < 8, the lo product of head c - 8
+            // otherwise; their sum, in both columns, is a row_ror:8 add)
+#pragma unroll
+            for (int i4 = 0; i4 < 4; ++i4) {
+                *reinterpret_cast<u4*>(kt + (kwr ^ (i4 << 6)) + 1024 * i4) = cur.k0[i4];
+                *reinterpret_cast<u4*>(kt + (kwr ^ (i4 << 6)) + 1024 * i4 + 4096) = cur.k1[i4];
+            }
+            k_free();                            // K is in LDS: its registers may be loaded again
             f4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
-            f4 t0 = {0.f, 0.f, 0.f, 0.f}, t1 = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int ks = 0; ks < 4; ++ks) {
-                const h8 ka = __builtin_bit_cast(h8, k_operand(cur.k0, ks));
-                const h8 kc = __builtin_bit_cast(h8, k_operand(cur.k1, ks));
-                const h8 qhi = __builtin_bit_cast(h8, s_q[kvh][ks][0][lane]);
-                const h8 qlo = __builtin_bit_cast(h8, s_q[kvh][ks][1][lane]);
-                s0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka, qhi, s0, 0, 0, 0);
-                s1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(kc, qhi, s1, 0, 0, 0);
-                t0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka, qlo, t0, 0, 0, 0);
-                t1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(kc, qlo, t1, 0, 0, 0);
+                const h8 ka = *reinterpret_cast<const h8*>(kt + (krd ^ (ks << 6)));
+                const h8 kc = *reinterpret_cast<const h8*>(kt + (krd ^ (ks << 6)) + 4096);
+                s0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka, q8[ks], s0, 0, 0, 0);
+                s1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(kc, q8[ks], s1, 0, 0, 0);
             }
-            s0 += t0;
-            s1 += t1;
+#pragma unroll
+            for (int ii = 0; ii < 4; ++ii) {
+                s0[ii] += swap_halves(s0[ii]);
+                s1[ii] += swap_halves(s1[ii]);
+            }
             float s[8];
             bool ok[8];
 #pragma unroll
@@ -759,14 +788,12 @@ decode_split_kernel(DecodeArgs a) {
                 m = mn;
             }
             float ps = 0.f;
-            h8 phi, plo;
+            h8 p8;                               // hi term for c < 8, lo term otherwise
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
                 const float p = ok[j] ? __builtin_amdgcn_exp2f(s[j] - m) : 0.f;
                 ps += p;
-                const _Float16 h = (_Float16)p;
-                phi[j] = h;
-                plo[j] = (_Float16)(p - (float)h);
+                p8[j] = (_Float16)fmaf(-(float)(_Float16)p, lo_col, p);
             }
             lsum += ps;
 
@@ -781,15 +808,12 @@ decode_split_kernel(DecodeArgs a) {
                 for (int u = 0; u < 4; ++u)
                     vw[u] = __builtin_amdgcn_perm(cur.v[2 * u + 1][cb >> 1], cur.v[2 * u][cb >> 1], sel);
                 const h8 va = __builtin_bit_cast(h8, vw);
-                acc[cb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(va, phi, acc[cb], 0, 0, 0);
-                acc[cb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(va, plo, acc[cb], 0, 0, 0);
+                acc[cb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(va, p8, acc[cb], 0, 0, 0);
             }
         };
 
-        // each wave keeps one pair (16 KiB) in flight; the 8 waves of the CU
-        // overlap each other's latency (measured: a second pair prefetched
-        // before the query conversion only delays the query rows further
-        // behind the chip's first burst, 0.778 -> 0.791 ms per config-2 step)
+        // (a second pair requested before the query conversion only delays the
+        // query rows: 24 short solo sessions 349 -> 378 us)
         if constexpr (kDB) {
             // the next pair's loads go out before this pair's arithmetic (two
             // pairs in flight per wave), so the wave's stream does not stop at
@@ -804,22 +828,51 @@ decode_split_kernel(DecodeArgs a) {
                 // issued before the waits for this pair (the counter drains in
                 // issue order): without the pin the scheduler sinks them below
                 __builtin_amdgcn_sched_barrier(0);
-                compute_pair(qp, cur);
+                compute_pair(qp, cur, [] {});
                 if (!m1) break;
                 const bool m2 = qp + 2 * RS < npairs;
                 load_pair(std::false_type{}, m2 ? qp + 2 * RS : qp, cur, m2);
                 __builtin_amdgcn_sched_barrier(0);
-                compute_pair(qp + RS, alt);
+                compute_pair(qp + RS, alt, [] {});
+            }
+        } else if constexpr (kAhead) {
+            // The next pair's K goes out as soon as this pair's is in LDS, its
+            // V when this pair's products are done: half a pair in flight per
+            // wave through the arithmetic, in no more registers (16 ragged 7B
+            // sessions, 28 layers: 793 -> 777 us; with one wave per kv head,
+            // whose 8 waves stream long ranges anyway, 676 -> 683 us on four
+            // 14B layers).  The last
+            // pair has a body of its own: loads under a condition would turn
+            // the waits at the loop's head into full drains, loads without
+            // effect cost the cache a pass each.
+            if (r < npairs) {
+                if (!early) load_pair(std::false_type{}, r, cur);
+                int qp = r;
+                for (; qp + RS < npairs; qp += RS) {
+                    const PagePair pp = pages_of(std::false_type{}, qp + RS);
+                    compute_pair(qp, cur, [&] {
+                        load_k(pp, cur);
+                        __builtin_amdgcn_sched_barrier(0);
+                    });
+                    load_v(pp, cur);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                compute_pair(qp, cur, [] {});
             }
         } else {
             for (int qp = r; qp < npairs; qp += RS) {
                 if (qp != r || !early) load_pair(std::false_type{}, qp, cur);
-                compute_pair(qp, cur);
+                compute_pair(qp, cur, [] {});
             }
         }
 
         lsum += shfl_xor_f(lsum, 16);
         lsum += shfl_xor_f(lsum, 32);
+        // O of head c: the products of the hi and of the lo weights
+#pragma unroll
+        for (int cb = 0; cb < 8; ++cb)
+#pragma unroll
+            for (int ii = 0; ii < 4; ++ii) acc[cb][ii] += swap_halves(acc[cb][ii]);
         // this wave's G rows of a partial slot, straight from the accumulators
         auto write_rows = [&](float* pout) {
             if (c < G) {
@@ -1031,10 +1084,8 @@ decode_stream_floor_kernel(DecodeArgs a) {
     const int pa = __builtin_amdgcn_readlane(hv, 1);
     const int pb = __builtin_amdgcn_readlane(hv, 2);
     const int32_t* table = a.tables + (int64_t)i * a.table_stride;
-    const uint32_t koff = (uint32_t)((c & 7) * kRowBytes + kvh * HD * 2 + 16 * (g + 4 * (c >> 3)));
-    uint32_t voff[4];
-#pragma unroll
-    for (int jj = 0; jj < 4; ++jj) voff[jj] = (uint32_t)((4 * g + jj) * kRowBytes + kvh * HD * 2 + 16 * c);
+    const uint32_t koff = (uint32_t)(g * kRowBytes + kvh * HD * 2 + 16 * c);
+    const uint32_t voff = (uint32_t)(4 * g * kRowBytes + kvh * HD * 2 + 16 * c);
     const char* pk = reinterpret_cast<const char*>(a.pool_k);
     const char* pv = reinterpret_cast<const char*>(a.pool_v);
     const int64_t layer_page0 = (int64_t)a.layer * a.nb;
@@ -1060,14 +1111,13 @@ decode_stream_floor_kernel(DecodeArgs a) {
         u4 x[16];
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks) {
-            const uint32_t o = koff + (ks & 1) * 8 * kRowBytes + (ks >> 1) * 128;
-            x[ks] = ldb16_nt(rk0, o);
-            x[4 + ks] = ldb16_nt(rk1, o);
+            x[ks] = ldb16_nt(rk0, koff, 4 * ks * kRowBytes);
+            x[4 + ks] = ldb16_nt(rk1, koff, 4 * ks * kRowBytes);
         }
 #pragma unroll
         for (int jj = 0; jj < 4; ++jj) {
-            x[8 + jj] = ldb16_nt(rv0, voff[jj]);
-            x[12 + jj] = ldb16_nt(rv1, voff[jj]);
+            x[8 + jj] = ldb16_nt(rv0, voff, jj * kRowBytes);
+            x[12 + jj] = ldb16_nt(rv1, voff, jj * kRowBytes);
         }
 #pragma unroll
         for (int e = 0; e < 16; ++e) sum += x[e];
@@ -1108,20 +1158,18 @@ decode_combine_kernel(DecodeArgs a, float* __restrict__ o) {
         pt.pages = e.w;
         pt.sess = i;
     } else {
-        if (a.kv_split) {
-            // single session: head kvh * G + m runs on a block whose XCD
-            // (t % 8) is congruent to kvh mod NKV, next to its split workgroups
-            constexpr int per8 = 8 / NKV;
-            const int x = t & 7, kv = x % NKV;
-            const int m = (t >> 3) * per8 + x / NKV;
-            if (m >= G) return;                  // padding block
-            i = 0;
-            h = kv * G + m;
-        } else {
-            i = t % a.n_sess;
-            h = t / a.n_sess;
-        }
-        pt = partition(a, 0, i);
+        // one session, kv-split: head kvh * G + m runs on a block whose XCD (t % 8)
+        // is congruent to kvh mod NKV, next to its split workgroups
+        constexpr int per8 = 8 / NKV;
+        const int x = t & 7, kv = x % NKV;
+        const int m = (t >> 3) * per8 + x / NKV;
+        if (m >= G) return;                      // padding block
+        i = 0;
+        h = kv * G + m;
+        pt.sess = 0;
+        pt.kc = 0;
+        pt.k = a.n_ranges;
+        pt.pages = a.n_pages;
     }
     f4* orow = reinterpret_cast<f4*>(o + ((int64_t)i * NH + h) * HD) + q4;
     if (pt.sess < 0 || pt.k == 0) {
@@ -1291,7 +1339,7 @@ decode_plan_kernel(DecodeArgs a, int32_t* __restrict__ plan) {
         return;
     }
     const int L = logical_of(w, xcd_stride(sum_k(a), a.gw), a.gw);
-    const Part pt = L >= 0 ? partition(a, L, -1) : Part{-1, 0, 0, 0, 0};
+    const Part pt = L >= 0 ? partition(a, L) : Part{-1, 0, 0, 0, 0};
     int32_t* rec = plan + plan_rec_off(a.n_sess) + (int64_t)w * kRec;
     if (pt.sess < 0) {
         if (lane == 0) rec[kRecPages] = -1;
@@ -1323,9 +1371,8 @@ int batch_workgroups() {
 }
 
 void launch_split(const DecodeArgs& a, int n_sess, hipStream_t st) {
-    const dim3 grid = a.kv_split ? dim3(NKV, a.gw + n_sess)
-                                 : dim3(a.plan ? split_slots(n_sess, a.gw) : a.gw + n_sess);
-    const bool single = a.plan && n_sess == 1;
+    const dim3 grid = a.kv_split ? dim3(NKV, a.n_ranges) : dim3(split_slots(n_sess, a.gw));
+    const bool single = n_sess == 1;
     if (a.kv_split) hipLaunchKernelGGL((decode_split_kernel<false, true>), grid, dim3(THREADS), 0, st, a);
     else if (a.cs && single) hipLaunchKernelGGL((decode_split_kernel<true, false, false, true>), grid, dim3(THREADS), 0, st, a);
     else if (a.cs) hipLaunchKernelGGL((decode_split_kernel<true, false>), grid, dim3(THREADS), 0, st, a);
@@ -1355,7 +1402,7 @@ void launch_solo(const DecodeArgs& a, int n_sess, hipStream_t st) {
 
 void launch_pair(const DecodeArgs& a, int n_sess, float* o, hipStream_t st) {
     launch_split(a, n_sess, st);
-    const int comb = a.plan ? n_sess * NH : a.kv_split ? 8 * ((NH + 7) / 8) : n_sess * NH;
+    const int comb = a.kv_split ? 8 * ((NH + 7) / 8) : n_sess * NH;
     hipLaunchKernelGGL(decode_combine_kernel, dim3(comb), dim3(CT), 0, st, a, o);
     NOVA_LAUNCHED();
 }
@@ -1556,10 +1603,11 @@ void launch_attn_decode_paged(const float* q, const uint16_t* pool_k, const uint
         return;
     }
     // scratch holds NH*32*(HD+2) floats (reference contract): at most 32
-    // partial slots, and the partition uses at most gw + 1 of them
+    // partial slots.  The partition of the one session is worked out here: in
+    // the kernels it cost 1.9 us before the first block-table entry was asked for.
     int gw = (pages + 1) / 2;
     if (gw > kMaxSplit - 1) gw = kMaxSplit - 1;
-    if (gw < 1) gw = 1;
+    const int share = share_of(pages, gw);
     DecodeArgs a{};
     a.q = q;
     a.pool_k = pool_k;
@@ -1572,7 +1620,8 @@ void launch_attn_decode_paged(const float* q, const uint16_t* pool_k, const uint
     a.layer = layer;
     a.nb = nb;
     a.part = scratch;
-    a.gw = gw;
+    a.n_pages = pages;
+    a.n_ranges = (pages + share - 1) / share;     // <= gw
     a.kv_split = 1;   // NKV workgroups per partial slot: 31 * NKV CUs per call
     a.spin = kSpinLimit;
     a.pw = PW;        // the reference's scratch holds NH*32*(HD+2) floats

@@ -469,3 +469,41 @@ def test_decode_rope_one_session(model, oracle):
     assert np.array_equal(gk, hk) and np.array_equal(gv, hv), "fused rope + append not bit-exact"
     ref = oracle.attn_decode_paged(model, np.ascontiguousarray(rq), hk, hv, tables[0], 0, fx.nb, int(n_keys[0]))
     assert_close(got[0], ref, what=f"{model} rope one session")
+
+
+@pytest.mark.parametrize("model", ["qwen25_7b", "qwen25_1p5b", "qwen25_14b"])
+@pytest.mark.parametrize("n_keys", [641, 656, 992, 993, 1985, 1999, 32225])
+def test_decode_single_page_ranges(model, n_keys, oracle):
+    """The one-session call past the one-launch limit (40 pages): its page
+    ranges at the edges of their split -- the first page count that splits, a
+    range of one page pair more or less, counts the ranges do not divide, and
+    ranges longer than the 64 table entries a wave holds (2015 pages over 31)."""
+    import nova_amd
+    nova = nova_amd.load(model)
+    print(f"[case] decode page ranges model={model} n_keys={n_keys}", flush=True)
+    pages = (n_keys + 15) // 16
+    fx = PagedFixture(nova, nb=pages + 3, layer=LAYER, seed=n_keys)
+    table = fx.tables(1, pages)[0]
+    q = fx.rng.standard_normal((nova.nh, nova.hd)).astype(np.float32)
+    got = _decode_single(nova, fx, q, table, n_keys)
+    err64 = float(np.abs(got - _decode_f64(q, fx.hk, fx.hv, table, n_keys, nova.group)).max())
+    assert err64 < 1e-4   # 2^-22 per operand over |v| < 6, with room for fp32 sums of 32225 terms
+
+
+@pytest.mark.parametrize("model", ["qwen25_7b", "qwen25_1p5b", "qwen25_14b"])
+def test_decode_batch_long_ranges(model, oracle):
+    """More sessions than workgroups, so each has one: page ranges of 65 to 70
+    pages, past the 64 table entries of a plan record, with 1 to 8 pairs left
+    for a wave's last round."""
+    import nova_amd
+    nova = nova_amd.load(model)
+    n, pages = 300, 70
+    print(f"[case] decode batch long ranges model={model}", flush=True)
+    fx = PagedFixture(nova, nb=pages + 3, layer=LAYER, seed=300)
+    tables = np.repeat(fx.tables(1, pages), n, axis=0)      # read-only, so all may share the pages
+    n_keys = (64 * 16 + 1 + np.arange(n) * 7 % 96).astype(np.int32)
+    q = fx.rng.standard_normal((n, nova.nh, nova.hd)).astype(np.float32)
+    got = _batch(nova, fx, q, tables, n_keys)
+    for i in range(0, n, 13):
+        ref = _decode_f64(q[i], fx.hk, fx.hv, tables[i], n_keys[i], nova.group)
+        assert np.abs(got[i] - ref).max() < 1e-4, f"session {i} n_keys={n_keys[i]}"
