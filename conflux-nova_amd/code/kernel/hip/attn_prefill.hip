@@ -17,9 +17,19 @@
 //    small launches also split the keys: their workgroups hold two groups of 4
 //    waves over the same columns, group g taking key tiles g, g+2, ..., each
 //    with its own LDS ring, and the two partial (O, l, m) are merged through
-//    LDS at the end (measured: one session's chunk 16% faster; with NB = 2
-//    the second group spills registers and is 26% slower, so wide launches
-//    keep one group).
+//    LDS at the end, each group taking half of the head dims (measured: one
+//    session's chunk 16% faster; with NB = 2 the second group spills registers
+//    and is 26% slower, so wide launches keep one group).
+//  * Rows in and out in address order.  The vector L1 takes one 128 B line of
+//    an instruction per clock, so 16 B per lane of 16 different rows cost it
+//    four times what lanes following each other along a row cost.  The output
+//    rows are turned in LDS before they are stored, and in small launches,
+//    whose few tiles do not hide it, the query rows are requested first, beside
+//    the block table, and turned in LDS while the first tiles load.  Per layer:
+//    a 173-token prompt of the 1.5B model 14.0 -> 11.6 us, a 512-token chunk
+//    behind 1536 of the 7B one 45.1 -> 42.8.  In wide launches the query
+//    rows' way through LDS would hold up the tiles: 426.2 us by it, 425.9
+//    without, for two layers of 8 sessions.
 //  * K/V tiles of 32 keys (2 pages) are staged ONCE per workgroup in LDS by
 //    direct global->LDS loads (global_load_lds_dwordx4: no staging
 //    registers), four buffers: while tile t's softmax runs, the scores of
@@ -326,7 +336,6 @@ prefill_kernel(PrefillArgs a) {
     __shared__ int32_t s_tab[kTabWin];
     static_assert((kBuckets + NT + 16) * 4 <= (int)sizeof(s_kv), "ranking scratch fits the tile buffers");
     static_assert(4 + NT / 64 <= 16 && kBuckets % NT == 0, "ranking scratch layout");
-    static_assert(KS == 1 || KS * 64 * NB * 34 * 4 * WAVES / KS <= (int)sizeof(s_kv), "merge scratch");
 
     const int tid = threadIdx.x;
     const int kg = tid / THREADS;                // key group
@@ -380,13 +389,46 @@ prefill_kernel(PrefillArgs a) {
     const uint32_t loff_k = (uint32_t)(srow * (KVW * 2) + 16 * schunk_k);
     const uint32_t loff_v = (uint32_t)(srow * (KVW * 2) + 16 * schunk_v);
     const uint32_t wave_s = __builtin_amdgcn_readfirstlane(wave);
+    // The workgroup's query rows, 16 B per lane along the rows, are requested
+    // before anything else and go through the last tile buffer of every group
+    // (free until step 0): chunk k of column q at position k ^ (q & 15) of its
+    // 512 B, no bank conflicts either way.  Only where the columns fit: with 128
+    // columns per key group every lane reads its own part of its row below.
+    constexpr int kQRow = HD * 4, kQGroup = STAGE_BYTES / kQRow;     // bytes of a row, columns per buffer
+    constexpr bool kStageQ = KS * kQGroup >= COLS_WG;
+    constexpr int kQLoads = kStageQ ? COLS_WG * HD / 4 / NT : 1;
+    static_assert(!kStageQ || COLS_WG * HD / 4 % NT == 0, "whole loads of the query rows");
+    auto q_row = [&](int col) -> const float* {              // a column past the last: row 0, unused
+        const int qi = col < n_cols ? col / G : 0;
+        return qs + ((int64_t)qi * NH + kvh * G + (col < n_cols ? col - qi * G : 0)) * HD;
+    };
+    auto s_q = [&](int q, int k) -> f4* {                    // q: column in the workgroup, k: 16 B chunk
+        return reinterpret_cast<f4*>(&s_kv[q / kQGroup][NBUF - 1][(q % kQGroup) * kQRow + ((k ^ (q & 15)) << 4)]);
+    };
+    f4 qraw[kQLoads];
+    if constexpr (kStageQ) {
+#pragma unroll
+        for (int e = 0; e < kQLoads; ++e) {
+            const int u = tid + e * NT;
+            qraw[e] = *reinterpret_cast<const f4*>(q_row(wg_col0 + u / (HD / 4)) + 4 * (u % (HD / 4)));
+        }
+    }
     int win0 = 0;                                            // first page of the LDS table window
-    auto load_window = [&](int first) {                      // every thread, uniform
+    auto load_window = [&](int first, auto&& with) {         // every thread, uniform
         for (int e = tid; e < kTabWin && first + e < n_pages; e += NT) s_tab[e] = table[first + e];
+        with();
         __syncthreads();
         win0 = first;
     };
-    load_window(0);
+    load_window(0, [&] {
+        if constexpr (kStageQ) {
+#pragma unroll
+            for (int e = 0; e < kQLoads; ++e) {
+                const int u = tid + e * NT;
+                *s_q(u / (HD / 4), u % (HD / 4)) = qraw[e];
+            }
+        }
+    });
     // physical pages of this group's tile of step i (tile KS*i + kg), read
     // from the LDS table a step before the loads that use them.  Every wave
     // calls this at the same points with the same i, so the window (which
@@ -396,7 +438,7 @@ prefill_kernel(PrefillArgs a) {
         const int pg_first = 2 * KS * i;                     // first page of step i's tiles
         if (pg_first < n_pages && pg_first + 2 * KS - 1 - win0 >= kTabWin) {
             __syncthreads();                                 // every wave is done with the old window
-            load_window(pg_first);
+            load_window(pg_first, [] {});
         }
         const int T = KS * i + kg;
         if (T >= n_tiles) return Pages{0, 0};                // no such tile for this group
@@ -453,15 +495,21 @@ prefill_kernel(PrefillArgs a) {
         const int col = col0 + 16 * b + c;
         const bool real = col < n_cols;
         const int qi = real ? col / G : 0;
-        const int hh = real ? col - qi * G : 0;
         qpos[b] = real ? n_past + qi : -1;
+        const int hh = real ? col - qi * G : 0;
         const float* qp = qs + ((int64_t)qi * NH + kvh * G + hh) * HD + 8 * g;
         float xv[4][8];
         float amax = 0.f;
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks) {
-            const f4 x0 = *reinterpret_cast<const f4*>(qp + 32 * ks);
-            const f4 x1 = *reinterpret_cast<const f4*>(qp + 32 * ks + 4);
+            f4 x0, x1;
+            if constexpr (kStageQ) {
+                x0 = *s_q(wave * COLS_WAVE + 16 * b + c, 8 * ks + 2 * g);
+                x1 = *s_q(wave * COLS_WAVE + 16 * b + c, 8 * ks + 2 * g + 1);
+            } else {
+                x0 = *reinterpret_cast<const f4*>(qp + 32 * ks);
+                x1 = *reinterpret_cast<const f4*>(qp + 32 * ks + 4);
+            }
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 xv[ks][j] = real ? x0[j] * (kScale * kLog2e) : 0.f;
@@ -488,6 +536,9 @@ prefill_kernel(PrefillArgs a) {
             }
         }
     }
+
+    // every lane has its query values: step 0 may load over them after the barrier
+    if constexpr (kStageQ) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
 
     // Running max m of the lane's column (log2 units); x = s - m is formed as
     // one fma of the raw (scaled) MFMA score with qf and -m.  m starts at 0;
@@ -687,46 +738,71 @@ prefill_kernel(PrefillArgs a) {
         lsum[b] += __shfl_xor(lsum[b], 32, 64);
     }
 
+    // ---- merge, normalise and store (the tile buffers are free: the last step
+    // ended with a barrier) ----
+    // Lane (g,c) of block b holds d = 16cb + 4g + i of its column.  With two key
+    // groups each keeps four of the eight cb: it hands the other four, its m and
+    // its l over through LDS and merges what it gets.
+    constexpr int CBN = 8 / KS;                              // cb this wave stores: [cb0, cb0 + CBN)
+    const int cb0 = KS == 2 ? CBN * kg : 0;
+    f4 out[NB][CBN];
     if constexpr (KS == 2) {
-        // merge group 1's (m, l, acc) into group 0's through LDS (the tile
-        // buffers are free: the last step ended with a barrier)
-        float* xs = reinterpret_cast<float*>(&s_kv[0][0][0]) + (wave * 64 + lane) * (NB * 34);
-        if (kg == 1) {
-#pragma unroll
-            for (int b = 0; b < NB; ++b) {
-#pragma unroll
-                for (int cb = 0; cb < 8; ++cb) *reinterpret_cast<f4*>(xs + b * 34 + 4 * cb) = acc[b][cb];
-                xs[b * 34 + 32] = lsum[b];
-                xs[b * 34 + 33] = m[b];
-            }
-        }
-        __syncthreads();
-        if (kg == 1) return;
+        f4* xo = reinterpret_cast<f4*>(&s_kv[0][0][0]);      // [kg][wave][NB][CBN][64]
+        float2* xm = reinterpret_cast<float2*>(&s_kv[0][0][0] + KS * WAVES * NB * CBN * 1024);   // [kg][wave][NB][64]
+        static_assert(KS * WAVES * NB * 64 * (CBN * 16 + 8) <= (int)sizeof(s_kv), "merge scratch");
+        const int mine = (kg * WAVES + wave) * NB, other = ((kg ^ 1) * WAVES + wave) * NB;
 #pragma unroll
         for (int b = 0; b < NB; ++b) {
-            const float l1 = xs[b * 34 + 32], m1 = xs[b * 34 + 33], l0 = lsum[b];
-            // a group without keys for this column has l = 0 and must not set the max
-            const float mm = l1 > 0.f ? (l0 > 0.f ? fmaxf(m[b], m1) : m1) : m[b];
-            const float f0 = l0 > 0.f ? __builtin_amdgcn_exp2f(m[b] - mm) : 0.f;
+#pragma unroll
+            for (int cb = 0; cb < CBN; ++cb) xo[((mine + b) * CBN + cb) * 64 + lane] = kg ? acc[b][cb] : acc[b][CBN + cb];
+            xm[(mine + b) * 64 + lane] = float2{lsum[b], m[b]};
+        }
+        __syncthreads();
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+            const float2 x = xm[(other + b) * 64 + lane];
+            // group 0 and group 1 in this order in both halves; a group without keys
+            // for this column has l = 0 and must not set the max
+            const float l0 = kg ? x.x : lsum[b], m0 = kg ? x.y : m[b], l1 = kg ? lsum[b] : x.x, m1 = kg ? m[b] : x.y;
+            const float mm = l1 > 0.f ? (l0 > 0.f ? fmaxf(m0, m1) : m1) : m0;
+            const float f0 = l0 > 0.f ? __builtin_amdgcn_exp2f(m0 - mm) : 0.f;
             const float f1 = l1 > 0.f ? __builtin_amdgcn_exp2f(m1 - mm) : 0.f;
 #pragma unroll
-            for (int cb = 0; cb < 8; ++cb)
-                acc[b][cb] = acc[b][cb] * f0 + *reinterpret_cast<const f4*>(xs + b * 34 + 4 * cb) * f1;
+            for (int cb = 0; cb < CBN; ++cb) {
+                const f4 o = xo[((other + b) * CBN + cb) * 64 + lane];
+                out[b][cb] = kg ? o * f0 + acc[b][CBN + cb] * f1 : acc[b][cb] * f0 + o * f1;
+            }
             lsum[b] = l0 * f0 + l1 * f1;
         }
+        __syncthreads();                                     // the rows below reuse the buffers
+    } else {
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+#pragma unroll
+            for (int cb = 0; cb < CBN; ++cb) out[b][cb] = acc[b][cb];
     }
-
-    // ---- normalise and store: lane (g,c) of block b holds d = 16cb + 4g + i ----
+    // The rows leave through a piece of LDS of the wave's own, so that a store's
+    // lanes follow each other along the rows: straight from the registers its 64
+    // lanes lie on 16 rows, which costs the vector L1 four times the clocks.
+    // Chunk k of row c sits at position k ^ c.
+    constexpr int RCH = 4 * CBN;                             // 16 B chunks per row
+    constexpr int RPS = 64 / RCH;                            // rows per store
+    static_assert(KS * WAVES * 16 * RCH * 16 <= (int)sizeof(s_kv), "store scratch");
+    f4* xr = reinterpret_cast<f4*>(&s_kv[0][0][0]) + (kg * WAVES + wave) * 16 * RCH;
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
-        const float L = lsum[b];
-        const int col = col0 + 16 * b + c;
-        if (col >= n_cols) continue;
-        const int qi = col / G, hh = col - qi * G;
-        float* op = os + ((int64_t)qi * NH + kvh * G + hh) * HD;
-        const float inv = 1.f / L;
+        const float inv = 1.f / lsum[b];
 #pragma unroll
-        for (int cb = 0; cb < 8; ++cb) *reinterpret_cast<f4*>(op + 16 * cb + 4 * g) = acc[b][cb] * inv;
+        for (int cb = 0; cb < CBN; ++cb) xr[c * RCH + ((4 * cb + g) ^ c)] = out[b][cb] * inv;
+#pragma unroll
+        for (int e = 0; e < CBN; ++e) {
+            const int row = RPS * e + lane / RCH, k = lane % RCH;
+            const f4 v = xr[row * RCH + (k ^ row)];
+            const int col = col0 + 16 * b + row;
+            if (col >= n_cols) continue;
+            const int qi = col / G, hh = col - qi * G;
+            *reinterpret_cast<f4*>(os + ((int64_t)qi * NH + kvh * G + hh) * HD + 16 * cb0 + 4 * k) = v;
+        }
     }
 }
 

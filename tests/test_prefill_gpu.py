@@ -231,3 +231,31 @@ def test_prefill_beyond_table_window(n_q, n_past):
     ref1 = _causal_f64(q[1], fx.hk, fx.hv, tables[1], n_q, 300, nova.group)
     assert_close(got[1], ref1, what="batched short session")
     print(f"  max|gpu-f64|={err:.3e}")
+
+
+@pytest.mark.parametrize("model,n_q", [
+    ("qwen25_7b", 9), ("qwen25_7b", 10), ("qwen25_7b", 18), ("qwen25_7b", 19),       # 63, 70, 126, 133 columns
+    ("qwen25_1p5b", 10), ("qwen25_1p5b", 11), ("qwen25_1p5b", 32), ("qwen25_1p5b", 33),     # 60, 66, 192, 198
+    ("qwen25_14b", 12), ("qwen25_14b", 13), ("qwen25_14b", 64),                      # 60, 65, 320
+])
+@pytest.mark.parametrize("n_past", [0, 15, 97])
+def test_prefill_column_edges(model, n_q, n_past, oracle):
+    """Column counts around whole workgroups of 64 (query rows and output rows
+    pass through LDS by columns), from one tile of keys, which leaves the second
+    key group without any, upwards; what lies past the output stays as it was."""
+    import nova_amd
+    nova = nova_amd.load(model)
+    print(f"[case] prefill edges model={model} n_q={n_q} n_past={n_past}", flush=True)
+    pages = (n_past + n_q + 15) // 16
+    fx = PagedFixture(nova, nb=pages + 4, layer=LAYER, seed=n_q + n_past)
+    table = fx.tables(1, pages)[0]
+    q = fx.rng.standard_normal((n_q, nova.nh, nova.hd)).astype(np.float32)
+    guard = np.full(4096, -7.5, np.float32)
+    dq, dt = nova.upload(q), nova.upload(table)
+    do = nova.upload(np.concatenate([np.zeros(q.size, np.float32), guard]))
+    nova.launch_attn_prefill_paged(dq.ptr, fx.k.ptr, fx.v.ptr, dt.ptr, LAYER, fx.nb, n_q, n_past, do.ptr, None)
+    nova.dev_sync()
+    got = do.numpy((q.size + guard.size,), np.float32)
+    assert np.array_equal(got[q.size:], guard)
+    ref = oracle.attn_prefill_paged(model, q, fx.hk, fx.hv, table, 0, fx.nb, n_q, n_past)
+    assert_close(got[:q.size].reshape(q.shape), ref, what=f"{model} n_q={n_q} n_past={n_past}")
