@@ -597,7 +597,8 @@ __global__ void __launch_bounds__(64 * kMaxKs4) gemv4_kernel(const uint8_t* __re
     const uint32_t xhalf = is_d ? 16 : 32;
     uint32_t buf = 0;                          // the unit being multiplied
     int to_come = n_units - 1;                 // units after it
-    f4 acc = {0.f, 0.f, 0.f, 0.f};             // tokens 0..3 of row c, sub-blocks 4h+g
+    // tokens 0..3 of row c, sub-blocks 4h+g; one sum per h: half as many roundings in a row
+    f4 acc2[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
     for (int b = 0; b < my; ++b) {
         for (int sb = sb_a; sb < sb_b; ++sb) {
             if (to_come > 0) {
@@ -635,11 +636,12 @@ __global__ void __launch_bounds__(64 * kMaxKs4) gemv4_kernel(const uint8_t* __re
                 const float dx[4] = {row_lane<0>(x), row_lane<1>(x), row_lane<2>(x), row_lane<3>(x)};
 #pragma unroll
                 for (int i = 0; i < 4; ++i)
-                    acc[i] += dx[i] * (al * (float)(g & 1 ? c1[i] : c0[i]) - bl * v[i]);
+                    acc2[h][i] += dx[i] * (al * (float)(g & 1 ? c1[i] : c0[i]) - bl * v[i]);
             }
             buf = kUnitBytes - buf;
         }
         // over the four groups of lanes, then with the other waves' after the barrier
+        f4 acc = acc2[0] + acc2[1];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(acc[i]), __float_as_uint(acc[i]), false, false);
@@ -648,7 +650,7 @@ __global__ void __launch_bounds__(64 * kMaxKs4) gemv4_kernel(const uint8_t* __re
             acc[i] = __uint_as_float(q[0]) + __uint_as_float(q[1]);
         }
         if (g == 0) s_part[((b & 1) * ks + wave) * 16 + c] = acc;
-        acc = f4{0.f, 0.f, 0.f, 0.f};
+        acc2[0] = acc2[1] = f4{0.f, 0.f, 0.f, 0.f};
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
@@ -750,9 +752,14 @@ void launch_quant_q8(int8_t* qs, float* d, int32_t* sums, const float* x, int ro
     NOVA_REQUIRE(qs && d && sums && x && rows >= 0 && cols > 0 && cols % 32 == 0);
     const int64_t n4 = (int64_t)rows * (cols / 4);
     if (n4 == 0) return;
-    hipLaunchKernelGGL(quant_kernel, dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, reinterpret_cast<hipStream_t>(s),
-                       qs, d, sums, x, n4);
-    NOVA_LAUNCHED();
+    // one launch takes fewer than 2^32 threads; whole blocks (8 pieces) per launch
+    constexpr int64_t kMost = (int64_t)1 << 31;
+    for (int64_t at = 0; at < n4; at += kMost) {
+        const int64_t n = n4 - at < kMost ? n4 - at : kMost;
+        hipLaunchKernelGGL(quant_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0,
+                           reinterpret_cast<hipStream_t>(s), qs + 4 * at, d + at / 8, sums + at / 4, x + 4 * at, n);
+        NOVA_LAUNCHED();
+    }
 }
 
 void launch_gemv_q4k(const uint8_t* blocks, int64_t rows, int cols, const int8_t* xq, const float* xd,
@@ -779,6 +786,15 @@ void launch_gemv4_q4k(const uint8_t* blocks, int64_t rows, int cols, const int8_
     NOVA_REQUIRE(cols > 0 && cols % kQK == 0 && cols <= kMaxCols4);
     NOVA_REQUIRE(aligned16(xq) && aligned16(xd) && aligned16(xs));   // staged with 16 B loads
     if (rows == 0) return;
+    // The direct loads to LDS move aligned 16 B; weights elsewhere (a file mapped
+    // at an odd offset) go token by token through the one-token kernel, whose
+    // register loads take any address: four weight reads instead of one.
+    if (!aligned16(blocks)) {
+        for (int t = 0; t < kTok4; ++t)
+            launch_gemv_q4k(blocks, rows, cols, xq + (int64_t)t * cols, xd + (int64_t)t * (cols / 32),
+                            xs + (int64_t)t * (cols / 16), out + t * rows, s);
+        return;
+    }
     launch_gemv4(blocks, rows, cols, xq, xd, xs, out, reinterpret_cast<hipStream_t>(s));
     NOVA_LAUNCHED();
 }

@@ -135,7 +135,7 @@ def test_gemv_f32_fused(cols, rows, nova7, oracle):
 
 @pytest.mark.parametrize("rows,cols", [(37, 256), (512, 3584), (3584, 3584), (130, 18944), (70, 8960),
                                        (33, 13824), (5, 28672), (1, 1536),
-                                       # 32M weights and up: the MFMA kernel (ragged 16-row blocks too)
+                                       # 32M weights and up (ragged 16-row blocks too)
                                        (2051, 16384), (20001, 2048), (18944, 3584), (3584, 18944)])
 def test_gemv4_matches_single_token(rows, cols, nova7, oracle):
     """launch_gemv4_q4k (4 stacked tokens, one weight read): every token's
@@ -178,3 +178,27 @@ def test_gemv4_edges(rows, cols, nova7, oracle):
     the widest rows, and more blocks than fit at once (a workgroup walks several,
     its last one ragged)."""
     test_gemv4_matches_single_token(rows, cols, nova7, oracle)
+
+
+@pytest.mark.parametrize("shift", [4, 8])
+@pytest.mark.parametrize("rows,cols", [(37, 256), (130, 3584), (33, 18944)])
+def test_gemv4_weights_off_16_bytes(rows, cols, shift, nova7, oracle):
+    """Weights that do not start on 16 B take the one-token kernel per token:
+    its bits for aligned weights, and nothing written past the output."""
+    nova = nova7
+    print(f"[case] gemv4 rows={rows} cols={cols} weights + {shift} B", flush=True)
+    rng = np.random.default_rng(rows + cols + shift)
+    w = np.ascontiguousarray(random_blocks(rng, rows, cols)).view(np.uint8).ravel()
+    x = rng.standard_normal((4, cols)).astype(np.float32)
+    dq, dd, ds = (nova.upload(a) for a in oracle.quant_q8(x))
+    aligned, shifted = nova.upload(w), nova.upload(np.concatenate([np.zeros(shift, np.uint8), w]))
+    out4 = nova.upload(np.full(4 * rows + 64, np.nan, np.float32))
+    one = nova.upload(np.full(4 * rows, np.nan, np.float32))
+    nova.launch_gemv4_q4k(shifted.ptr + shift, rows, cols, dq.ptr, dd.ptr, ds.ptr, out4.ptr, None)
+    for t in range(4):
+        nova.launch_gemv_q4k(aligned.ptr, rows, cols, dq.ptr + t * cols, dd.ptr + t * (cols // 32) * 4,
+                             ds.ptr + t * (cols // 16) * 4, one.ptr + t * rows * 4, None)
+    nova.dev_sync()
+    got, ref = out4.numpy((4 * rows + 64,), np.float32), one.numpy((4 * rows,), np.float32)
+    assert np.array_equal(got[:4 * rows].view(np.uint32), ref.view(np.uint32))
+    assert np.all(np.isnan(got[4 * rows:]))
