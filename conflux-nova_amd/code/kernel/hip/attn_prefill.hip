@@ -236,16 +236,18 @@ __device__ int lpt_item(const PrefillArgs& a, int r, int n_cg, int n_cols, int c
 // disjoint.  The pipeline waits for these loads explicitly (tile_barrier);
 // the compiler's waits for its own loads stay correct, as the counter drains
 // in issue order.  m0 is a register the compiler reserves (it cannot be
-// declared clobbered), so the statement saves and restores it.
+// declared clobbered), so the statement saves and restores it.  An LDS load
+// needs one wait state after a scalar write of m0, which neither the hardware
+// nor, inside a statement, the compiler supplies: s_nop 0.
 __device__ __forceinline__ void dma16x4(const void* s0, const void* s1, const void* s2, const void* s3,
                                         uint32_t lds) {
     uint32_t saved;
     asm volatile(
         "s_mov_b32 %0, m0\n\t"
-        "s_mov_b32 m0, %5\n\tglobal_load_lds_dwordx4 %1, off\n\t"
-        "s_mov_b32 m0, %6\n\tglobal_load_lds_dwordx4 %2, off\n\t"
-        "s_mov_b32 m0, %7\n\tglobal_load_lds_dwordx4 %3, off\n\t"
-        "s_mov_b32 m0, %8\n\tglobal_load_lds_dwordx4 %4, off\n\t"
+        "s_mov_b32 m0, %5\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off\n\t"
+        "s_mov_b32 m0, %6\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, off\n\t"
+        "s_mov_b32 m0, %7\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %3, off\n\t"
+        "s_mov_b32 m0, %8\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %4, off\n\t"
         "s_mov_b32 m0, %0"
         : "=&s"(saved)
         : "v"(s0), "v"(s1), "v"(s2), "v"(s3), "s"(lds), "s"(lds + 16u * THREADS), "s"(lds + 32u * THREADS),
@@ -262,10 +264,10 @@ __device__ __forceinline__ void dma16x4_s(const void* k0, const void* k1, const 
     uint32_t saved;
     asm volatile(
         "s_mov_b32 %0, m0\n\t"
-        "s_mov_b32 m0, %7\n\tglobal_load_lds_dwordx4 %5, %1\n\t"
-        "s_mov_b32 m0, %8\n\tglobal_load_lds_dwordx4 %5, %2\n\t"
-        "s_mov_b32 m0, %9\n\tglobal_load_lds_dwordx4 %6, %3\n\t"
-        "s_mov_b32 m0, %10\n\tglobal_load_lds_dwordx4 %6, %4\n\t"
+        "s_mov_b32 m0, %7\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %5, %1\n\t"
+        "s_mov_b32 m0, %8\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %5, %2\n\t"
+        "s_mov_b32 m0, %9\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %6, %3\n\t"
+        "s_mov_b32 m0, %10\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %6, %4\n\t"
         "s_mov_b32 m0, %0"
         : "=&s"(saved)
         : "s"(k0), "s"(k1), "s"(v0), "s"(v1), "v"(off_k), "v"(off_v), "s"(lds), "s"(lds + 16u * THREADS),

@@ -431,8 +431,10 @@ __global__ void __launch_bounds__(QT) gemv_split_kernel(GemvSet g) {
 // Direct global -> LDS loads: the wave's 64 pieces of 16 B go to the 1 KiB at
 // LDS byte address lds.  Inline asm, so that the compiler's vmcnt bookkeeping
 // does not see them (it would drain them before every LDS read it cannot prove
-// disjoint); wave_wait waits for them.  m0 cannot be declared clobbered, so the
-// statement saves and restores it.
+// disjoint); gemv4_kernel waits for them.  m0 cannot be declared clobbered, so
+// the statement saves and restores it.  An LDS load needs one wait state after a
+// scalar write of m0, which neither the hardware nor, inside a statement, the
+// compiler supplies: s_nop 0.
 __device__ __forceinline__ void stream_load(const void* base, uint32_t off, uint32_t lds) {
     // wave-uniform base: kept in scalar registers whatever the compiler made of it
     const uint64_t b = (uint64_t)base;
@@ -441,7 +443,7 @@ __device__ __forceinline__ void stream_load(const void* base, uint32_t off, uint
     uint32_t saved;
     asm volatile(
         "s_mov_b32 %0, m0\n\t"
-        "s_mov_b32 m0, %3\n\tglobal_load_lds_dwordx4 %2, %1\n\t"
+        "s_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %1\n\t"
         "s_mov_b32 m0, %0"
         : "=&s"(saved)
         : "s"(sb), "v"(off), "s"(lds)
@@ -453,7 +455,7 @@ __device__ __forceinline__ void stream_load_at(const void* p, uint32_t lds) {
     uint32_t saved;
     asm volatile(
         "s_mov_b32 %0, m0\n\t"
-        "s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %1, off\n\t"
+        "s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off\n\t"
         "s_mov_b32 m0, %0"
         : "=&s"(saved)
         : "v"(p), "s"(lds)
