@@ -259,17 +259,21 @@ __device__ __forceinline__ void dma16x4(const void* s0, const void* s1, const vo
 // page bases in SGPR pairs (K page 0, K page 1, V page 0, V page 1) and the
 // lane's 32-bit offsets inside a page (one for K, one for V), so the loop
 // keeps two offset registers instead of four 64-bit addresses per tile.
+// A vector memory instruction needs five wait states after a vector instruction
+// wrote its base (a v_readlane of a block table, say).  A scalar copy waits for
+// such a write by itself and may be read at once, and it is m0's wait state too.
 __device__ __forceinline__ void dma16x4_s(const void* k0, const void* k1, const void* v0, const void* v1,
                                           uint32_t off_k, uint32_t off_v, uint32_t lds) {
     uint32_t saved;
+    uint64_t base;
     asm volatile(
         "s_mov_b32 %0, m0\n\t"
-        "s_mov_b32 m0, %7\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %5, %1\n\t"
-        "s_mov_b32 m0, %8\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %5, %2\n\t"
-        "s_mov_b32 m0, %9\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %6, %3\n\t"
-        "s_mov_b32 m0, %10\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %6, %4\n\t"
+        "s_mov_b32 m0, %8\n\ts_mov_b64 %1, %2\n\tglobal_load_lds_dwordx4 %6, %1\n\t"
+        "s_mov_b32 m0, %9\n\ts_mov_b64 %1, %3\n\tglobal_load_lds_dwordx4 %6, %1\n\t"
+        "s_mov_b32 m0, %10\n\ts_mov_b64 %1, %4\n\tglobal_load_lds_dwordx4 %7, %1\n\t"
+        "s_mov_b32 m0, %11\n\ts_mov_b64 %1, %5\n\tglobal_load_lds_dwordx4 %7, %1\n\t"
         "s_mov_b32 m0, %0"
-        : "=&s"(saved)
+        : "=&s"(saved), "=&s"(base)
         : "s"(k0), "s"(k1), "s"(v0), "s"(v1), "v"(off_k), "v"(off_v), "s"(lds), "s"(lds + 16u * THREADS),
           "s"(lds + 32u * THREADS), "s"(lds + 48u * THREADS)
         : "memory");

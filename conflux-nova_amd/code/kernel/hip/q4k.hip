@@ -434,18 +434,22 @@ __global__ void __launch_bounds__(QT) gemv_split_kernel(GemvSet g) {
 // disjoint); gemv4_kernel waits for them.  m0 cannot be declared clobbered, so
 // the statement saves and restores it.  An LDS load needs one wait state after a
 // scalar write of m0, which neither the hardware nor, inside a statement, the
-// compiler supplies: s_nop 0.
+// compiler supplies.
 __device__ __forceinline__ void stream_load(const void* base, uint32_t off, uint32_t lds) {
-    // wave-uniform base: kept in scalar registers whatever the compiler made of it
+    // wave-uniform base: kept in scalar registers whatever the compiler made of
+    // it.  A vector memory instruction needs five wait states after v_readfirstlane
+    // wrote its base; a scalar copy waits for such a write by itself and may be
+    // read at once, and it is m0's wait state too.
     const uint64_t b = (uint64_t)base;
     const uint64_t sb = ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(b >> 32)) << 32) |
                         (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)b);
     uint32_t saved;
+    uint64_t copy;
     asm volatile(
         "s_mov_b32 %0, m0\n\t"
-        "s_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %1\n\t"
+        "s_mov_b32 m0, %4\n\ts_mov_b64 %1, %2\n\tglobal_load_lds_dwordx4 %3, %1\n\t"
         "s_mov_b32 m0, %0"
-        : "=&s"(saved)
+        : "=&s"(saved), "=&s"(copy)
         : "s"(sb), "v"(off), "s"(lds)
         : "memory");
 }

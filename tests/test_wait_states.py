@@ -39,22 +39,26 @@ def _instructions(lib, tmp_path):
     for n, obj in enumerate(_code_objects(lib)):
         path = tmp_path / f"{lib.stem}_{n}.co"
         path.write_bytes(obj)
-        text = subprocess.run([OBJDUMP, "-d", "--no-show-raw-insn", str(path)], capture_output=True, text=True,
-                              check=True).stdout
-        name, code = None, []
-        for line in text.splitlines():
-            head = re.match(r"[0-9a-f]+ <(.+)>:$", line)
-            if head:
-                if code:
-                    yield name, code
-                name, code = head[1], []
-                continue
-            line = line.split("//")[0].strip()
-            if name and line:
-                op, _, rest = line.partition(" ")
-                code.append((op, rest.strip()))
-        if code:
-            yield name, code
+        yield from _disassemble(path)
+
+
+def _disassemble(path):
+    text = subprocess.run([OBJDUMP, "-d", "--no-show-raw-insn", str(path)], capture_output=True, text=True,
+                          check=True).stdout
+    name, code = None, []
+    for line in text.splitlines():
+        head = re.match(r"[0-9a-f]+ <(.+)>:$", line)
+        if head:
+            if code:
+                yield name, code
+            name, code = head[1], []
+            continue
+        line = line.split("//")[0].strip()
+        if name and line:
+            op, _, rest = line.partition(" ")
+            code.append((op, rest.strip()))
+    if code:
+        yield name, code
 
 
 def _registers(operand):
@@ -118,3 +122,65 @@ def test_lds_loads_after_m0(model, tmp_path):
             lambda op: op.startswith("s_"), 1)]
     assert loads >= 16                            # the search sees the prefill and the four-token kernels
     assert not found, f"{len(found)} of {loads} loads:\n" + "\n".join(found[:10])
+
+
+def _scalar_base_hazards(code):
+    def bases(op, rest):
+        if not op.startswith(("global_", "buffer_", "flat_", "scratch_")):
+            return set()
+        return {r for t in _operands(rest) for r in _registers(t) if r[0] == "s"}
+    return _missing(code, bases, lambda op: op.startswith("v_"), 5)
+
+
+# A base that comes straight from a vector register: the worst a caller can do.
+PROBES = {
+    "q4k": """
+        extern "C" __global__ void probe(const uint64_t* p, uint32_t lds) {
+            nova::stream_load((const void*)p[threadIdx.x], 16 * threadIdx.x, lds);
+        }""",
+    "attn_prefill": """
+        extern "C" __global__ void probe(const uint64_t* p, uint32_t lds) {
+            const uint64_t b = p[threadIdx.x];
+            const void* base = (const void*)((uint64_t)__builtin_amdgcn_readfirstlane((uint32_t)(b >> 32)) << 32 |
+                                             (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)b));
+            nova::dma16x4_s(base, base, base, base, 16 * threadIdx.x, 16 * threadIdx.x, lds);
+        }""",
+}
+
+
+@pytest.mark.parametrize("source", sorted(PROBES))
+def test_scalar_bases_from_vector_registers(source, tmp_path):
+    """A vector memory instruction needs five wait states after a vector
+    instruction wrote the scalar registers of its base.  The direct loads are
+    compiled here behind v_readfirstlane."""
+    from pathlib import Path
+    import build as nova_build
+    src = tmp_path / "probe.hip"
+    src.write_text(f'#include "{Path(nova_build.PKG) / "code/kernel/hip" / (source + ".hip")}"\n{PROBES[source]}\n')
+    out = tmp_path / "probe.co"
+    subprocess.run([nova_build.HIPCC, *nova_build.COMMON, *nova_build.HIP_FLAGS, "-DNOVA_MODEL_QWEN25_7B",
+                    "--offload-device-only", "--no-gpu-bundle-output", "-c", str(src), "-o", str(out)], check=True,
+                   capture_output=True)
+    code = dict(_disassemble(out))["probe"]
+    assert any(_is_lds_load(op, rest) for op, rest in code)
+    assert any(op == "v_readfirstlane_b32" for op, _ in code)
+    found = _scalar_base_hazards(code) + _missing(
+        code, lambda op, rest: {("m0", 0)} if _is_lds_load(op, rest) else set(), lambda op: op.startswith("s_"), 1)
+    assert not found, "\n".join(found)
+
+
+@pytest.mark.parametrize("model", ["qwen25_1p5b", "qwen25_7b", "qwen25_14b"])
+def test_scalar_bases_in_the_libraries(model, tmp_path):
+    """The same in the built libraries, and one wait state between a vector
+    register's write and its read by v_readlane or v_readfirstlane (the decode
+    kernel settles a load's result in a statement of its own before such reads)."""
+    import nova_amd
+
+    def lanes(op, rest):
+        return _registers(_operands(rest)[1]) if op in ("v_readlane_b32", "v_readfirstlane_b32") else set()
+    found = []
+    for lib in (nova_amd.lib_path(model), nova_amd.testkit_path(model)):
+        for kernel, code in _instructions(lib, tmp_path):
+            for m in _scalar_base_hazards(code) + _missing(code, lanes, lambda op: op.startswith("v_"), 1):
+                found.append(f"{kernel}: {m}")
+    assert not found, "\n".join(found[:10])
