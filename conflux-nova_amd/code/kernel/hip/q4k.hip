@@ -666,17 +666,184 @@ __global__ void __launch_bounds__(64 * kMaxKs4) gemv4_kernel(const uint8_t* __re
     }
 }
 
+// ---------------------------------------------------------------- four tokens, weights anywhere
+// Weights that do not start on 16 B (a file mapped at an odd offset) cannot take
+// the direct loads.  Here they are read into registers, once for the four
+// tokens, with the one-token kernels' lanes, steps and order of sums: the bits
+// are those of launch_gemv_q4k for each token.
+//
+// Bound by LDS reads of the activations, one row against four of them.  The
+// codes therefore lie in four planes per token, chunk q of every quarter
+// super-block in plane q: a read's 64 lanes take 1 KiB without bank conflicts,
+// where the one-token layout's 64 B between lanes cost this kernel half its time
+// (18944 x 3584: 22.5 us, in planes 13.9); the scale and the sum of a 32 sit
+// side by side, one read for both sub-blocks.  A row's first loads go out before
+// the activations are staged.  The four sums of a row share their cross-lane
+// steps (wave_sums4).  Workgroups of 512 threads; with 1024, a CU holds fewer of
+// a narrow launch's waves (5120 x 5120: 11.3 us against 9.5).
+// us per launch, weights at + 4 B / + 1 B, against four one-token launches:
+// 512 x 3584 3.8 / 4.2 (12.2 / 12.9), 3584 x 3584 6.0 / 6.5 (16.9 / 19.2),
+// 18944 x 3584 13.9 / 15.9 (34.9 / 42.5), 3584 x 18944 16.9 / 18.0 (39.0 / 43.8),
+// 5120 x 13824 19.6 / 22.5 (41.0 / 48.7), 152064 x 3584 82 / 97 (226 / 338).  The
+// direct loads, on 16 B: 3.7, 4.5, 11.6, 12.4, 15.7, 75.
+
+// One token's products of a lane's share: chunk q of four (16 codes: sub-block 2c
+// q = 0, 1; sub-block 2c + 1 q = 2, 3) at sq + q * plane, scale and sum of both
+// sub-blocks in ds.  The combination is sb_dot's.
+__device__ __forceinline__ float sb_dot_planes(const SbW& w, const int8_t* sq, int plane, const f4 ds) {
+    int dlo = 0, dhi = 0;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const i4 alo = *reinterpret_cast<const i4*>(sq + h * plane);
+        const i4 ahi = *reinterpret_cast<const i4*>(sq + (2 + h) * plane);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            dlo = __builtin_amdgcn_sdot4(alo[e], w.lo[4 * h + e], dlo, false);
+            dhi = __builtin_amdgcn_sdot4(ahi[e], w.hi[4 * h + e], dhi, false);
+        }
+    }
+    return ds[0] * (w.al * (float)dlo - w.bl * ds[1]) + ds[2] * (w.ah * (float)dhi - w.bh * ds[3]);
+}
+
+// Four ActQ8 activations into LDS: codes as four planes per token (chunk q of
+// every quarter super-block), scale and sum of each 32 side by side.  No barrier.
+template <int NT>
+__device__ __forceinline__ void stage_planes4(const int8_t* xq, const float* xd, const int32_t* xs, int cols, int8_t* s_q,
+                                              float2* s_ds) {
+    const int per = cols / 16, n = kTok4 * per, nd = kTok4 * (cols / 32);
+    constexpr int NQ = 4;
+    for (int b = threadIdx.x; b < n; b += NQ * NT) {
+        u4 v[NQ];
+        float d[NQ];
+        int2 sm[NQ];
+        const int bd = b - (int)threadIdx.x;
+#pragma unroll
+        for (int k = 0; k < NQ; ++k) {
+            if (b + k * NT < n) v[k] = *reinterpret_cast<const u4*>(xq + 16 * (b + k * NT));
+            if (k < NQ / 2) {
+                const int e = bd / 2 + (int)threadIdx.x + k * NT;
+                if (e < nd) {
+                    d[k] = xd[e];
+                    sm[k] = *reinterpret_cast<const int2*>(xs + 2 * e);
+                }
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < NQ; ++k) {
+            const int u = b + k * NT, t = u / per, i = u - t * per;
+            if (u < n) *reinterpret_cast<u4*>(s_q + t * cols + (i & 3) * (cols / 4) + (i >> 2) * 16) = v[k];
+            if (k < NQ / 2) {
+                const int e = bd / 2 + (int)threadIdx.x + k * NT;
+                if (e < nd) s_ds[e] = float2{d[k], (float)(sm[k].x + sm[k].y)};
+            }
+        }
+    }
+}
+
+// Sums of four values over the 64 lanes, in __shfl_xor's order 32, 16, 8, 4, 2, 1;
+// lane 16t gets the sum of a[t'], t' = (t >> 1) | (t & 1) << 1.
+__device__ __forceinline__ float wave_sums4(const float* a) {
+    float h[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {             // lanes < 32: a[2i], others: a[2i + 1]
+        const auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(a[2 * i]), __float_as_uint(a[2 * i + 1]), false, false);
+        h[i] = __uint_as_float(p[0]) + __uint_as_float(p[1]);
+    }
+    const auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(h[0]), __float_as_uint(h[1]), false, false);
+    float v = __uint_as_float(p[0]) + __uint_as_float(p[1]);
+    v += dpp_f<0x128>(v);                      // row_ror:8: lane ^ 8
+    v += dpp_f<0x104>(v);                      // row_shl:4: lanes 0..3 of a row
+    v += dpp_f<kXor2>(v);
+    return v + dpp_f<kXor1>(v);
+}
+
+// STEPS and KS as in gemv_fixed_kernel (KS == 1) and gemv_split_kernel, whose
+// fourth wave per row has nothing below 97 super-blocks: KS == 3 there.
+template <int STEPS, int KS, int NT>
+__global__ void __launch_bounds__(NT) gemv4_rows_kernel(const uint8_t* __restrict__ w, int64_t rows, int cols,
+                                                        const int8_t* __restrict__ xq, const float* __restrict__ xd,
+                                                        const int32_t* __restrict__ xs, float* __restrict__ out) {
+    static_assert(NT % (64 * KS) == 0, "whole rows per workgroup");
+    constexpr int RPI = NT / 64 / KS;          // rows per workgroup iteration
+    // the next row's loads behind this row's unpacking; with more steps the
+    // registers cost more waves than that hides (1536 x 8960: 7.9 us, 7.6 without)
+    constexpr bool kAhead = STEPS == 1 || KS > 1;
+    extern __shared__ __attribute__((aligned(16))) unsigned char s_x[];
+    __shared__ float s_part[2][KS > 1 ? NT / 64 : 1][kTok4];
+    int8_t* s_q = reinterpret_cast<int8_t*>(s_x);                        // [4 tokens][4 planes][cols/4]
+    float2* s_ds = reinterpret_cast<float2*>(s_x + kTok4 * cols);        // [4][cols/32]
+
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int part = wave % KS;
+    const int j = lane / kLps, c = lane % kLps;
+    const int nsb = cols / kQK;
+    const int sb0 = kSbPerStep * STEPS * part + j;
+    const int64_t row_bytes = (int64_t)nsb * kBlockBytes;
+    const int64_t stride = (int64_t)gridDim.x * RPI;
+
+    u4 hdr[STEPS];
+    Nib nib[STEPS];
+    auto load = [&](int64_t r, int t) {        // a wave past the end: the last row, unused
+        const int sb = sb0 + kSbPerStep * t;
+        if (sb >= nsb) return;
+        const uint8_t* blk = w + (r < rows ? r : rows - 1) * row_bytes + (int64_t)sb * kBlockBytes;
+        hdr[t] = *reinterpret_cast<const u4*>(blk);
+        nib[t] = load_nib(blk, c);
+    };
+    int64_t r = (int64_t)blockIdx.x * RPI + wave / KS;
+#pragma unroll
+    for (int t = 0; t < STEPS; ++t) load(r, t);
+    stage_planes4<NT>(xq, xd, xs, cols, s_q, s_ds);
+    __syncthreads();
+    int parity = 0;
+    // the same number of rounds for every wave of the workgroup
+    for (int64_t base = (int64_t)blockIdx.x * RPI; base < rows; base += stride, r += stride) {
+        float acc[kTok4] = {0.f, 0.f, 0.f, 0.f};
+        const bool more = base + stride < rows;
+#pragma unroll
+        for (int t = 0; t < STEPS; ++t) {
+            const int sb = sb0 + kSbPerStep * t;
+            const SbW wv = sb_prep(hdr[t], nib[t], c);
+            if (kAhead && more) load(r + stride, t);
+            if (sb < nsb)
+#pragma unroll
+                for (int k = 0; k < kTok4; ++k)
+                    acc[k] += sb_dot_planes(wv, s_q + k * cols + 16 * (4 * sb + c), cols / 4,
+                                            *reinterpret_cast<const f4*>(s_ds + k * (cols / 32) + 8 * sb + 2 * c));
+        }
+        if (!kAhead && more)
+#pragma unroll
+            for (int t = 0; t < STEPS; ++t) load(r + stride, t);
+        const float v = wave_sums4(acc);
+        const int tok = (lane >> 5) | (lane >> 4 & 1) << 1;
+        if constexpr (KS == 1) {
+            if ((lane & 15) == 0 && r < rows) out[tok * rows + r] = v;
+        } else {
+            if ((lane & 15) == 0) s_part[parity][wave][tok] = v;
+            __syncthreads();
+            if (part == 0 && lane < kTok4 && r < rows) {
+                float sum = s_part[parity][wave][lane];
+#pragma unroll
+                for (int p = 1; p < KS; ++p) sum += s_part[parity][wave + p][lane];
+                out[lane * rows + r] = sum;
+            }
+            parity ^= 1;                       // the next write here comes after the next barrier
+        }
+    }
+}
+
 // Workgroups: one per rows_per_wg rows, but no more than can be resident at
 // once (this kernel's occupancy at this LDS size times the CUs); beyond that
 // the kernels grid-stride, so no second partial round of workgroups forms a
 // tail (measured: gate projection 9.8 -> 9.0 us against a fixed cap of 8
 // workgroups per CU, of which 7 fit).
 template <typename K>
-int gemv_grid(K kernel, int64_t rows, int rows_per_wg, size_t lds) {
+int gemv_grid(K kernel, int64_t rows, int rows_per_wg, size_t lds, int block = QT) {
     int dev = 0, cus = 0, per_cu = 0;
     NOVA_HIP(hipGetDevice(&dev));
     NOVA_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-    NOVA_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, QT, lds));
+    NOVA_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, block, lds));
     if (per_cu < 1) per_cu = 1;
     const int64_t want = (rows + rows_per_wg - 1) / rows_per_wg;
     const int64_t cap = (int64_t)per_cu * cus;
@@ -727,6 +894,20 @@ void launch_gemv4(const uint8_t* blocks, int64_t rows, int cols, const int8_t* x
     const int grid = (int)(n_rb < cap ? n_rb : cap);
     hipLaunchKernelGGL(gemv4_kernel, dim3(grid), dim3(64 * ks), lds_of(ks), s, blocks, rows, cols, xq, xd, xs, out,
                        (int)(n_rb / grid), (int)(n_rb % grid));
+}
+
+template <int STEPS, int KS, int NT>
+void launch_rows4(const uint8_t* blocks, int64_t rows, int cols, const int8_t* xq, const float* xd, const int32_t* xs,
+                  float* out, hipStream_t s) {
+    auto k = gemv4_rows_kernel<STEPS, KS, NT>;
+    static std::once_flag once;                // dynamic LDS beyond 64 KB must be allowed per kernel
+    std::call_once(once, [&] {
+        NOVA_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                     kTok4 * kMaxCols4 * 5 / 4));
+    });
+    const size_t lds = kTok4 * ((size_t)cols + 8 * (size_t)(cols / 32));
+    hipLaunchKernelGGL(k, dim3((unsigned)gemv_grid(k, rows, NT / 64 / KS, lds, NT)), dim3(NT), lds, s, blocks, rows, cols,
+                       xq, xd, xs, out);
 }
 
 template <bool kF32>
@@ -792,13 +973,20 @@ void launch_gemv4_q4k(const uint8_t* blocks, int64_t rows, int cols, const int8_
     NOVA_REQUIRE(cols > 0 && cols % kQK == 0 && cols <= kMaxCols4);
     NOVA_REQUIRE(aligned16(xq) && aligned16(xd) && aligned16(xs));   // staged with 16 B loads
     if (rows == 0) return;
-    // The direct loads to LDS move aligned 16 B; weights elsewhere (a file mapped
-    // at an odd offset) go token by token through the one-token kernel, whose
-    // register loads take any address: four weight reads instead of one.
+    // the direct loads to LDS move aligned 16 B; loads to registers take any address
     if (!aligned16(blocks)) {
-        for (int t = 0; t < kTok4; ++t)
-            launch_gemv_q4k(blocks, rows, cols, xq + (int64_t)t * cols, xd + (int64_t)t * (cols / 32),
-                            xs + (int64_t)t * (cols / 16), out + t * rows, s);
+        const hipStream_t st = reinterpret_cast<hipStream_t>(s);
+        switch ((cols / kQK + kSbPerStep - 1) / kSbPerStep) {      // launch_set's shapes, for its order of sums
+            case 1: launch_rows4<1, 1, 512>(blocks, rows, cols, xq, xd, xs, out, st); break;
+            case 2: launch_rows4<2, 1, 512>(blocks, rows, cols, xq, xd, xs, out, st); break;
+            case 3: launch_rows4<3, 1, 512>(blocks, rows, cols, xq, xd, xs, out, st); break;
+            case 4: launch_rows4<4, 1, 512>(blocks, rows, cols, xq, xd, xs, out, st); break;
+            // 12 waves: one workgroup fits a CU's LDS (3584 x 18944: 9 waves 17.3 us, 12 16.9, 15 16.8;
+            // 9000 x 18944: 34.0, 31.4, 34.5)
+            case 5: case 6: launch_rows4<2, 3, 768>(blocks, rows, cols, xq, xd, xs, out, st); break;
+            default: launch_rows4<2, 4, 768>(blocks, rows, cols, xq, xd, xs, out, st); break;     // 7: kMaxCols4
+        }
+        NOVA_LAUNCHED();
         return;
     }
     launch_gemv4(blocks, rows, cols, xq, xd, xs, out, reinterpret_cast<hipStream_t>(s));

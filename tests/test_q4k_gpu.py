@@ -202,3 +202,53 @@ def test_gemv4_weights_off_16_bytes(rows, cols, shift, nova7, oracle):
     got, ref = out4.numpy((4 * rows + 64,), np.float32), one.numpy((4 * rows,), np.float32)
     assert np.array_equal(got[:4 * rows].view(np.uint32), ref.view(np.uint32))
     assert np.all(np.isnan(got[4 * rows:]))
+
+
+@pytest.mark.parametrize("rows,cols,shift", [(1, 256, 1), (9, 4096, 2), (7, 4352, 1), (520, 8192, 4), (20, 8448, 12),
+                                             (9, 12544, 8), (17, 16384, 1), (4, 16640, 4), (13, 24576, 2),
+                                             (5, 24832, 8), (1030, 28672, 4), (9301, 1024, 4)])
+def test_gemv4_off_16_bytes_edges(rows, cols, shift, nova7, oracle):
+    """Rows of whole and broken steps of 16 super-blocks, both sides of each
+    change of steps and of waves per row, workgroups that are not full, and more
+    rows than are resident at once; weights at any byte."""
+    test_gemv4_weights_off_16_bytes(rows, cols, shift, nova7, oracle)
+
+
+@pytest.mark.parametrize("rows,cols", [(18944, 3584), (3584, 18944)])
+def test_gemv4_off_16_bytes_reads_weights_once(rows, cols, nova7):
+    """Four tokens over weights off 16 B cost less than 2.5 one-token launches
+    over the same weights: 1.3 and 1.5 where the weights are read once, 4 where
+    the call is four of them."""
+    nova = nova7
+    print(f"[case] gemv4 one read rows={rows} cols={cols}", flush=True)
+    n = rows * (cols // 256) * 144
+    copies = 10                                # more than the last-level cache holds
+    rng = np.random.default_rng(rows)
+    w = nova.upload(rng.integers(0, 64, copies * n + 16, dtype=np.uint8))
+    xq = nova.upload(rng.integers(-127, 128, (4, cols), dtype=np.int8))
+    xd = nova.upload(np.ones((4, cols // 32), np.float32))
+    xs = nova.upload(np.zeros((4, cols // 16), np.int32))
+    out = nova.alloc(4 * rows * 4)
+    stream = nova.dev_stream_create()
+    start, stop = nova.dev_event_create(), nova.dev_event_create()
+
+    def us(launch):
+        nova.dev_graph_begin(stream)
+        for c in range(copies):
+            launch(w.ptr + c * n + 4, rows, cols, xq.ptr, xd.ptr, xs.ptr, out.ptr, stream)
+        graph = nova.dev_graph_end(stream)
+        took = []
+        for _ in range(10):
+            nova.dev_event_record(start, stream)
+            nova.dev_graph_launch(graph, stream)
+            nova.dev_event_record(stop, stream)
+            took.append(nova.dev_event_elapsed_ms(start, stop))
+        nova.dev_graph_destroy(graph)
+        return min(took) * 1e3 / copies
+
+    one, four = us(nova.launch_gemv_q4k), us(nova.launch_gemv4_q4k)
+    print(f"  one token {one:.2f} us, four {four:.2f} us")
+    nova.dev_event_destroy(start)
+    nova.dev_event_destroy(stop)
+    nova.dev_stream_destroy(stream)
+    assert four < 2.5 * one
