@@ -147,13 +147,13 @@ __device__ __forceinline__ float half_to_float(uint32_t h) {
 // get_scale_min_k4, q4_k.h:44-52, for sub-block j of the 12 scale bytes
 // held as three little-endian words
 __device__ __forceinline__ void scale_min(int j, const uint32_t sw[3], uint32_t& sc, uint32_t& m) {
-    auto byte = [&](int k) -> uint32_t { return (sw[k >> 2] >> (8 * (k & 3))) & 0xFFu; };
+    const uint32_t b0 = sw[0] >> (8 * (j & 3)), b1 = sw[1] >> (8 * (j & 3)), b2 = sw[2] >> (8 * (j & 3));
     if (j < 4) {
-        sc = byte(j) & 63;
-        m = byte(j + 4) & 63;
+        sc = b0 & 63;
+        m = b1 & 63;
     } else {
-        sc = (byte(j + 4) & 0xF) | ((byte(j - 4) >> 6) << 4);
-        m = (byte(j + 4) >> 4) | ((byte(j) >> 6) << 4);
+        sc = (b2 & 0xF) | ((b0 >> 6 & 3) << 4);
+        m = (b2 >> 4 & 0xF) | ((b1 >> 6 & 3) << 4);
     }
 }
 
