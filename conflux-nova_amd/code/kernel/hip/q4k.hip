@@ -683,7 +683,7 @@ __global__ void __launch_bounds__(64 * kMaxKs4) gemv4_kernel(const uint8_t* __re
 // a narrow launch's waves (5120 x 5120: 11.3 us against 9.5).
 // us per launch, weights at + 4 B / + 1 B, against four one-token launches:
 // 512 x 3584 3.8 / 4.2 (12.2 / 12.9), 3584 x 3584 6.0 / 6.5 (16.9 / 19.2),
-// 18944 x 3584 13.9 / 15.9 (34.9 / 42.5), 3584 x 18944 16.9 / 18.0 (39.0 / 43.8),
+// 18944 x 3584 13.5 / 15.9 (34.9 / 42.5), 3584 x 18944 16.9 / 18.0 (39.0 / 43.8),
 // 5120 x 13824 19.6 / 22.5 (41.0 / 48.7), 152064 x 3584 82 / 97 (226 / 338).  The
 // direct loads, on 16 B: 3.7, 4.5, 11.6, 12.4, 15.7, 75.
 
@@ -758,7 +758,8 @@ __device__ __forceinline__ float wave_sums4(const float* a) {
 }
 
 // STEPS and KS as in gemv_fixed_kernel (KS == 1) and gemv_split_kernel, whose
-// fourth wave per row has nothing below 97 super-blocks: KS == 3 there.
+// fourth wave per row has nothing below 97 super-blocks: KS == 3 there.  Aligned
+// weights of few rows, whose order of sums is free, also with STEPS == 1, KS > 1.
 template <int STEPS, int KS, int NT>
 __global__ void __launch_bounds__(NT) gemv4_rows_kernel(const uint8_t* __restrict__ w, int64_t rows, int cols,
                                                         const int8_t* __restrict__ xq, const float* __restrict__ xd,
@@ -863,6 +864,13 @@ void launch_split(const GemvSet& g, size_t lds, hipStream_t s) {
     hipLaunchKernelGGL(k, dim3((unsigned)gemv_grid(k, g.end[g.n - 1], 1, lds)), dim3(QT), lds, s, g);
 }
 
+int device_cus() {
+    int dev = 0, cus = 0;
+    NOVA_HIP(hipGetDevice(&dev));
+    NOVA_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+    return cus;
+}
+
 // Waves per 16-row block: the fewest rounds of resident workgroups (LDS bounds
 // them) times the units that each of their waves takes, and among equals the
 // fewest waves: more of them only split the sums further.  Within 4% of the best
@@ -873,9 +881,7 @@ void launch_gemv4(const uint8_t* blocks, int64_t rows, int cols, const int8_t* x
     std::call_once(once, [&] {
         NOVA_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(gemv4_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, kLdsMax));
     });
-    int dev = 0, cus = 0;
-    NOVA_HIP(hipGetDevice(&dev));
-    NOVA_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+    const int cus = device_cus();
     auto lds_of = [](int k) { return (size_t)k * (2 * kUnitBytes + 16 + 2 * 16 * 16); };
     const int64_t n_rb = (rows + 15) / 16;
     const int nsb = cols / kQK;
@@ -908,6 +914,14 @@ void launch_rows4(const uint8_t* blocks, int64_t rows, int cols, const int8_t* x
     const size_t lds = kTok4 * ((size_t)cols + 8 * (size_t)(cols / 32));
     hipLaunchKernelGGL(k, dim3((unsigned)gemv_grid(k, rows, NT / 64 / KS, lds, NT)), dim3(NT), lds, s, blocks, rows, cols,
                        xq, xd, xs, out);
+}
+
+// rows of more than 64 super-blocks.  12 waves: one workgroup fits a CU's LDS
+// (3584 x 18944: 9 waves 17.3 us, 12 16.9, 15 16.8; 9000 x 18944: 34.0, 31.4, 34.5)
+void launch_rows4_wide(const uint8_t* blocks, int64_t rows, int cols, const int8_t* xq, const float* xd,
+                       const int32_t* xs, float* out, hipStream_t s) {
+    if (cols / kQK <= 6 * kSbPerStep) launch_rows4<2, 3, 768>(blocks, rows, cols, xq, xd, xs, out, s);
+    else launch_rows4<2, 4, 768>(blocks, rows, cols, xq, xd, xs, out, s);
 }
 
 template <bool kF32>
@@ -973,23 +987,32 @@ void launch_gemv4_q4k(const uint8_t* blocks, int64_t rows, int cols, const int8_
     NOVA_REQUIRE(cols > 0 && cols % kQK == 0 && cols <= kMaxCols4);
     NOVA_REQUIRE(aligned16(xq) && aligned16(xd) && aligned16(xs));   // staged with 16 B loads
     if (rows == 0) return;
-    // the direct loads to LDS move aligned 16 B; loads to registers take any address
+    const hipStream_t st = reinterpret_cast<hipStream_t>(s);
+    const int steps = (cols / kQK + kSbPerStep - 1) / kSbPerStep;
     if (!aligned16(blocks)) {
-        const hipStream_t st = reinterpret_cast<hipStream_t>(s);
-        switch ((cols / kQK + kSbPerStep - 1) / kSbPerStep) {      // launch_set's shapes, for its order of sums
+        // the direct loads to LDS move aligned 16 B; loads to registers take any address
+        switch (steps) {                       // launch_set's shapes, for its order of sums
             case 1: launch_rows4<1, 1, 512>(blocks, rows, cols, xq, xd, xs, out, st); break;
             case 2: launch_rows4<2, 1, 512>(blocks, rows, cols, xq, xd, xs, out, st); break;
             case 3: launch_rows4<3, 1, 512>(blocks, rows, cols, xq, xd, xs, out, st); break;
             case 4: launch_rows4<4, 1, 512>(blocks, rows, cols, xq, xd, xs, out, st); break;
-            // 12 waves: one workgroup fits a CU's LDS (3584 x 18944: 9 waves 17.3 us, 12 16.9, 15 16.8;
-            // 9000 x 18944: 34.0, 31.4, 34.5)
-            case 5: case 6: launch_rows4<2, 3, 768>(blocks, rows, cols, xq, xd, xs, out, st); break;
-            default: launch_rows4<2, 4, 768>(blocks, rows, cols, xq, xd, xs, out, st); break;     // 7: kMaxCols4
+            default: launch_rows4_wide(blocks, rows, cols, xq, xd, xs, out, st); break;
         }
-        NOVA_LAUNCHED();
-        return;
+    } else if (steps > 2 && (rows + 15) / 16 <= device_cus() / 4) {
+        // Few rows, and long ones: the 16-row blocks would leave three CUs of four
+        // idle while their 16 waves take more than two units each, one after the
+        // other.  By rows, every wave or three or four of them on a row of its own:
+        // 1024 x 20480 8.8 us (16-row blocks 11.6), 512 x 18944 7.5 (10.6), 1024 x
+        // 14336 6.5 (9.1), 512 x 10240 4.6 (5.9), 130 x 18944 6.4 (8.0).  Past that
+        // line the blocks win: 1536 x 8960 6.8 us, by rows 7.3.
+        switch (steps) {
+            case 3: launch_rows4<1, 3, 768>(blocks, rows, cols, xq, xd, xs, out, st); break;
+            case 4: launch_rows4<1, 4, 1024>(blocks, rows, cols, xq, xd, xs, out, st); break;
+            default: launch_rows4_wide(blocks, rows, cols, xq, xd, xs, out, st); break;
+        }
+    } else {
+        launch_gemv4(blocks, rows, cols, xq, xd, xs, out, st);
     }
-    launch_gemv4(blocks, rows, cols, xq, xd, xs, out, reinterpret_cast<hipStream_t>(s));
     NOVA_LAUNCHED();
 }
 

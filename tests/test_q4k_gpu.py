@@ -214,15 +214,12 @@ def test_gemv4_off_16_bytes_edges(rows, cols, shift, nova7, oracle):
     test_gemv4_weights_off_16_bytes(rows, cols, shift, nova7, oracle)
 
 
-@pytest.mark.parametrize("rows,cols", [(18944, 3584), (3584, 18944)])
-def test_gemv4_off_16_bytes_reads_weights_once(rows, cols, nova7):
-    """Four tokens over weights off 16 B cost less than 2.5 one-token launches
-    over the same weights: 1.3 and 1.5 where the weights are read once, 4 where
-    the call is four of them."""
-    nova = nova7
-    print(f"[case] gemv4 one read rows={rows} cols={cols}", flush=True)
+def _gemv_us(nova, rows, cols, calls):
+    """us per launch of each (entry point, shift): the shortest of ten replays
+    over copies of the weights, `shift` bytes off 16, that the last-level cache
+    does not hold."""
     n = rows * (cols // 256) * 144
-    copies = 10                                # more than the last-level cache holds
+    copies = max(10, -(-380_000_000 // n))
     rng = np.random.default_rng(rows)
     w = nova.upload(rng.integers(0, 64, copies * n + 16, dtype=np.uint8))
     xq = nova.upload(rng.integers(-127, 128, (4, cols), dtype=np.int8))
@@ -231,11 +228,11 @@ def test_gemv4_off_16_bytes_reads_weights_once(rows, cols, nova7):
     out = nova.alloc(4 * rows * 4)
     stream = nova.dev_stream_create()
     start, stop = nova.dev_event_create(), nova.dev_event_create()
-
-    def us(launch):
+    us = []
+    for launch, shift in calls:
         nova.dev_graph_begin(stream)
         for c in range(copies):
-            launch(w.ptr + c * n + 4, rows, cols, xq.ptr, xd.ptr, xs.ptr, out.ptr, stream)
+            launch(w.ptr + c * n + shift, rows, cols, xq.ptr, xd.ptr, xs.ptr, out.ptr, stream)
         graph = nova.dev_graph_end(stream)
         took = []
         for _ in range(10):
@@ -244,11 +241,42 @@ def test_gemv4_off_16_bytes_reads_weights_once(rows, cols, nova7):
             nova.dev_event_record(stop, stream)
             took.append(nova.dev_event_elapsed_ms(start, stop))
         nova.dev_graph_destroy(graph)
-        return min(took) * 1e3 / copies
-
-    one, four = us(nova.launch_gemv_q4k), us(nova.launch_gemv4_q4k)
-    print(f"  one token {one:.2f} us, four {four:.2f} us")
+        us.append(min(took) * 1e3 / copies)
     nova.dev_event_destroy(start)
     nova.dev_event_destroy(stop)
     nova.dev_stream_destroy(stream)
+    return us
+
+
+@pytest.mark.parametrize("rows,cols", [(18944, 3584), (3584, 18944)])
+def test_gemv4_off_16_bytes_reads_weights_once(rows, cols, nova7):
+    """Four tokens over weights off 16 B cost less than 2.5 one-token launches
+    over the same weights: 1.3 and 1.5 where the weights are read once, 4 where
+    the call is four of them."""
+    nova = nova7
+    print(f"[case] gemv4 one read rows={rows} cols={cols}", flush=True)
+    one, four = _gemv_us(nova, rows, cols, [(nova.launch_gemv_q4k, 4), (nova.launch_gemv4_q4k, 4)])
+    print(f"  one token {one:.2f} us, four {four:.2f} us")
     assert four < 2.5 * one
+
+
+@pytest.mark.parametrize("rows,cols", [(512, 18944), (1024, 20480)])
+def test_gemv4_few_long_rows_are_spread(rows, cols, nova7):
+    """Weights on 16 B are not slower than the same off 16 B, also where there
+    are too few 16-row blocks for the chip: 1.0 times as long, 1.3 and 1.4 with
+    the blocks' kernel."""
+    nova = nova7
+    print(f"[case] gemv4 few long rows rows={rows} cols={cols}", flush=True)
+    on, off = _gemv_us(nova, rows, cols, [(nova.launch_gemv4_q4k, 0), (nova.launch_gemv4_q4k, 4)])
+    print(f"  on 16 B {on:.2f} us, off {off:.2f} us")
+    assert on < 1.15 * off
+
+
+@pytest.mark.parametrize("rows,cols", [(1, 8448), (1024, 8448), (1025, 8448), (1024, 8192), (7, 12288), (1024, 12544),
+                                       (1025, 12544), (5, 16384), (1023, 16640), (1025, 16640), (14, 24576), (9, 24832),
+                                       (1024, 28672)])
+def test_gemv4_few_long_rows(rows, cols, nova7, oracle):
+    """Both sides of the lines between the kernel by rows and the one by 16-row
+    blocks (33 super-blocks, 1024 rows on 256 CUs) and of its changes of waves
+    per row, against the oracle and the one-token kernel."""
+    test_gemv4_matches_single_token(rows, cols, nova7, oracle)
