@@ -1132,10 +1132,16 @@ decode_stream_floor_kernel(DecodeArgs a) {
 // (attn.cu:163-191): M = max m_s, L = sum over l_s > 0 of l_s*2^(m_s-M),
 // O = sum acc_s*2^(m_s-M) / L; a session without keys gets O = 0.  Its 8
 // groups of 32 threads (a thread owns 4 consecutive head-dim columns) take
-// every 8th slot, 8 slots per group with all loads in flight, and the 8 group
-// results are merged through LDS by the same rule.  Measured against one
+// every 8th slot, 2, 4 or 8 slots per group with all loads in flight, and the 8
+// group results are merged through LDS by the same rule.  Measured against one
 // workgroup per (session, kv head) walking all slots: 448 instead of 64
-// workgroups for config 2, 0.876 -> 0.859 ms per step.
+// workgroups for config 2, 0.876 -> 0.859 ms per step.  Bound by one memory
+// latency: the row's place comes from a product instead of a division, no load
+// sits behind a branch or another load's arithmetic, and no more spare rows are
+// read than needed.  Split + combine per layer against rounds of 8 as the
+// compiler ordered them, us: 32 sessions of 100 to 500 keys 12.4 -> 11.4 (1.5B),
+// 16.3 -> 14.5 (7B), 19.1 -> 16.9 (14B); 4 of 8000 keys 19.5 -> 18.2 (1.5B); 16 of
+// 512 to 8192 34.9 -> 34.1 (7B); one of 1024 keys 13.4 -> 12.9 (14B).
 static_assert(8 % NKV == 0, "kv heads must divide the 8 XCDs");
 constexpr int CT = 256;                       // combine threads
 constexpr int kCombGroups = CT / (HD / 4);
@@ -1185,43 +1191,58 @@ decode_combine_kernel(DecodeArgs a, float* __restrict__ o) {
     const int stride = a.wave_parts == 1 ? R : 1;
     const int used = a.wave_parts == 1 ? min(R, (range_max_pages(pt.pages, pt.k) + 1) >> 1) : 1;
     const int n_rows = pt.k * used;
+    // sl / used as a product: exact below 2^14 rows, 8 divisions less ahead of the loads
+    static_assert(R <= 4, "per_used covers 1 to 4 rows");
+    const uint32_t per_used = used == 1 ? 65536u : used == 2 ? 32768u : used == 3 ? 21846u : 16384u;
     const float* base = a.part + (int64_t)pt.kc * stride * SEG + (int64_t)h * a.pw;
     float M = -INFINITY, L = 0.f;
     f4 A = {0.f, 0.f, 0.f, 0.f};
-    for (int s0 = g; s0 < n_rows; s0 += kCombGroups * kChunk) {
-        float ms[kChunk], ls[kChunk];
-        f4 as[kChunk];
+    auto merge = [&](auto rows_tag, int s0) {        // rows s0, s0 + kCombGroups, ... of this group
+        constexpr int N = decltype(rows_tag)::value;
+        float ms[N], ls[N];
+        f4 as[N];
+        const int spare = s0 < n_rows ? s0 : 0;      // read in place of a row past the last
 #pragma unroll
-        for (int jj = 0; jj < kChunk; ++jj) {
+        for (int jj = 0; jj < N; ++jj) {
             const int sl0 = s0 + jj * kCombGroups;
-            const bool in = sl0 < n_rows;
-            const int sl = in ? sl0 : s0;
-            const int wg = sl / used;
-            const float* row = base + (int64_t)(wg * stride + (sl - wg * used)) * SEG;
+            const int sl = sl0 < n_rows ? sl0 : spare;
+            const int wg = (int)(((uint32_t)sl * per_used) >> 16);
+            const float* row = base + (int64_t)(sl + wg * (stride - used)) * SEG;
             ms[jj] = row[0];
-            ls[jj] = in ? row[1] : 0.f;
+            ls[jj] = row[1];
             as[jj] = *reinterpret_cast<const f4*>(row + a.po + 4 * q4);
         }
+        // all loads in flight before the first wait: left to itself the compiler
+        // moves some behind the exponentials of others, a memory latency more
+        __builtin_amdgcn_sched_barrier(0);
         float mc = M;
 #pragma unroll
-        for (int jj = 0; jj < kChunk; ++jj)
+        for (int jj = 0; jj < N; ++jj) {
+            ls[jj] = s0 + jj * kCombGroups < n_rows ? ls[jj] : 0.f;
             if (ls[jj] > 0.f) mc = fmaxf(mc, ms[jj]);
+        }
         const float rescale = L > 0.f ? exp2f(M - mc) : 0.f;
         L *= rescale;
         A *= rescale;
 #pragma unroll
-        for (int jj = 0; jj < kChunk; ++jj) {
+        for (int jj = 0; jj < N; ++jj) {
             const float f = ls[jj] > 0.f ? exp2f(ms[jj] - mc) : 0.f;
             L = fmaf(ls[jj], f, L);
             A += as[jj] * f;
         }
         M = mc;
-    }
+    };
+    // rows past the last are loaded for nothing: no more of them than needed
+    int first = 0;
+    for (; n_rows - first > 4 * kCombGroups; first += kChunk * kCombGroups)
+        merge(std::integral_constant<int, kChunk>{}, first + g);
+    if (n_rows - first > 2 * kCombGroups) merge(std::integral_constant<int, 4>{}, first + g);
+    else if (n_rows > first) merge(std::integral_constant<int, 2>{}, first + g);
     if (q4 == 0) {
         s_m[g] = M;
         s_l[g] = L;
     }
-    s_a[g][q4] = A;
+    s_a[g][q4] = L > 0.f ? A : f4{0.f, 0.f, 0.f, 0.f};      // nothing of a spare row, whatever it holds
     __syncthreads();
     if (g != 0) return;
     float Mx = -INFINITY;

@@ -507,3 +507,25 @@ def test_decode_batch_long_ranges(model, oracle):
     for i in range(0, n, 13):
         ref = _decode_f64(q[i], fx.hk, fx.hv, tables[i], n_keys[i], nova.group)
         assert np.abs(got[i] - ref).max() < 1e-4, f"session {i} n_keys={n_keys[i]}"
+
+
+@pytest.mark.parametrize("model", ["qwen25_7b", "qwen25_1p5b", "qwen25_14b"])
+@pytest.mark.parametrize("pages", [(1, 4), (63, 64, 65), (127, 128, 129), (255, 257), (271, 289), (385, 513)])
+def test_decode_combine_rounds(model, pages):
+    """Sessions whose partial rows end on both sides of a round of the combine:
+    a workgroup of the split takes four pages or more, so these have 1 to 17, 32,
+    33, 64 to 73, 97 and 129 rows (times the waves with a slot of their own)."""
+    import nova_amd
+    nova = nova_amd.load(model)
+    print(f"[case] decode combine rounds model={model} pages={pages}", flush=True)
+    n_keys = np.array([16 * p - 5 for p in pages], np.int32)
+    fx = PagedFixture(nova, nb=sum(pages) + 3, layer=LAYER, seed=sum(pages))
+    perm = fx.rng.permutation(fx.nb).astype(np.int32)
+    tables = np.zeros((len(pages), max(pages)), np.int32)
+    for i, p in enumerate(pages):
+        tables[i, :p] = perm[sum(pages[:i]):sum(pages[:i]) + p]
+    q = fx.rng.standard_normal((len(pages), nova.nh, nova.hd)).astype(np.float32)
+    got = _batch(nova, fx, q, tables, n_keys)
+    for i, n in enumerate(n_keys):
+        err = np.abs(got[i] - _decode_f64(q[i], fx.hk, fx.hv, tables[i], int(n), nova.group)).max()
+        assert err < 3e-6, f"{n} keys: {err:.2e}"      # operands to 2^-22, fp32 sums; 1e-4 would pass for fp16 queries

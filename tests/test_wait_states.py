@@ -184,3 +184,21 @@ def test_scalar_bases_in_the_libraries(model, tmp_path):
             for m in _scalar_base_hazards(code) + _missing(code, lanes, lambda op: op.startswith("v_"), 1):
                 found.append(f"{kernel}: {m}")
     assert not found, "\n".join(found[:10])
+
+
+@pytest.mark.parametrize("model", ["qwen25_1p5b", "qwen25_7b", "qwen25_14b"])
+def test_combine_loads_go_out_together(model, tmp_path):
+    """Each round of the decode combine (2, 4 or 8 rows of a maximum, a sum and
+    4 accumulators per thread) has all its loads in flight before the first wait
+    for one of them: the launch lasts as long as its memory latencies in a row."""
+    import nova_amd
+    found = [code for kernel, code in _instructions(nova_amd.lib_path(model), tmp_path) if "decode_combine" in kernel]
+    assert len(found) == 1
+    rounds, run = [], 0
+    for op, rest in found[0]:
+        if op.startswith("global_load"):
+            run += 1
+        elif op == "s_waitcnt" and "vmcnt" in rest and run:
+            rounds.append(run)
+            run = 0
+    assert sorted(rounds) == [4, 8, 16]
