@@ -393,8 +393,12 @@ decode_split_kernel(DecodeArgs a) {
     // the wave index, and with it the pair loop and the page resources, in scalar
     // registers; not in a single session's step, whose waves take about one pair
     // each and have nothing to gain from it (28 1.5B layers of
-    // 1040 keys: 274 us against 279 with it and 286 before K went through LDS)
-    constexpr bool kUniform = !kSingle;
+    // 1040 keys: 274 us against 279 with it and 286 before K went through LDS),
+    // nor with four waves per kv head (1.5B), whose ranges are as short (us per
+    // layer, in scalar registers and without: 4 x 500-2000 keys 11.0, 10.8; 8 x
+    // 500-2000 12.2, 11.8; 13 x 196-1730 13.0, 12.7; 16 x 2000-8000 24.4, 24.4;
+    // 8 x 32000 51.8, 52.0)
+    constexpr bool kUniform = kKvSplit || (R < 4 && !kSingle);
     const int wave = kUniform ? __builtin_amdgcn_readfirstlane(tid >> 6) : tid >> 6;
     const int lane = tid & 63;
     const int g = lane >> 4;      // 0..3
