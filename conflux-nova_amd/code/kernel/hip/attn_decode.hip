@@ -1409,12 +1409,14 @@ void launch_split(const DecodeArgs& a, int n_sess, hipStream_t st) {
 // Solo launch: grid (kv head, session), the output written by the split
 // kernel.  Up to this many pages the reference-signature decode runs as one
 // solo launch instead of the split + combine pair.  Measured per layer (the
-// reference's launch_kv_store_paged + launch_attn_decode_paged, graph of 28
-// layers): 64 tokens 7.9 vs 14.4 us, 512 tokens 12.3 vs 14.2 us, 768 tokens
-// 14.8 vs 14.3 us (1.5B; 7B alike).  One CU's arithmetic, ~2.3 us per round
-// of one page pair per wave, is what limits a solo workgroup.
+// reference's launch_rope_kv_store_paged + launch_attn_decode_paged, graph of 28
+// layers), solo against pair, us for 1.5B / 7B / 14B: 64 keys 7.7 / 8.2 / 8.5
+// against 10.1 / 10.9 / 11.0, 320 keys 9.7 / 10.5 / 10.6 against 10.3 / 11.1 /
+// 11.7, 384 keys 10.3 / 11.2 / 11.3 against 10.3 / 11.0 / 11.8, 448 keys 10.9 /
+// 11.9 / 12.1 against 10.4 / 11.5 / 11.8, 640 keys 12.4 / 13.6 / 13.8 against
+// 10.5 / 11.6 / 12.0.  What limits a solo workgroup is one CU's arithmetic.
 #ifndef NOVA_DECODE_SOLO_PAGES
-#define NOVA_DECODE_SOLO_PAGES 40
+#define NOVA_DECODE_SOLO_PAGES 24
 #endif
 constexpr int kSoloMaxPages = NOVA_DECODE_SOLO_PAGES;
 void launch_solo(const DecodeArgs& a, int n_sess, hipStream_t st) {

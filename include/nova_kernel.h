@@ -146,7 +146,8 @@ void launch_attn_decode_paged_rope_batch(const float* q, const float* k_new, con
  * suits steps whose sessions hold up to about 40 pages (640 tokens); longer
  * sessions belong on the split path (on config 1's single 1025-key session
  * the split path is faster).  The reference's launch_attn_decode_paged takes
- * this route itself for contexts up to 40 pages.  The _rope_ form fuses RoPE
+ * this route itself for contexts up to 24 pages (384 tokens), where it beats
+ * that call's own split.  The _rope_ form fuses RoPE
  * as launch_attn_decode_paged_rope_planned does. */
 void launch_attn_decode_paged_solo(const float* q, uint16_t* pool_k, uint16_t* pool_v, const int32_t* tables,
                                    int table_stride, const int32_t* n_keys, int n_sess, int layer, int nb,

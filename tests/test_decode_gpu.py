@@ -472,12 +472,13 @@ def test_decode_rope_one_session(model, oracle):
 
 
 @pytest.mark.parametrize("model", ["qwen25_7b", "qwen25_1p5b", "qwen25_14b"])
-@pytest.mark.parametrize("n_keys", [641, 656, 992, 993, 1985, 1999, 32225])
+@pytest.mark.parametrize("n_keys", [369, 384, 385, 400, 449, 512, 640, 641, 656, 992, 993, 1985, 1999, 32225])
 def test_decode_single_page_ranges(model, n_keys, oracle):
-    """The one-session call past the one-launch limit (40 pages): its page
-    ranges at the edges of their split -- the first page count that splits, a
-    range of one page pair more or less, counts the ranges do not divide, and
-    ranges longer than the 64 table entries a wave holds (2015 pages over 31)."""
+    """The one-session call around and past the one-launch limit (24 pages): its
+    page ranges at the edges of their split -- the last page count of one launch
+    and the first that splits, a range of one page pair more or less, counts the
+    ranges do not divide, and ranges longer than the 64 table entries a wave
+    holds (2015 pages over 31)."""
     import nova_amd
     nova = nova_amd.load(model)
     print(f"[case] decode page ranges model={model} n_keys={n_keys}", flush=True)

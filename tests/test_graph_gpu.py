@@ -242,7 +242,7 @@ def test_gemv4_mfma_graph(nova7):
 def test_reference_call_pattern_graph(nova7):
     """the reference's per-session calls (launch_kv_store_paged, then
     launch_attn_decode_paged) for sessions on both sides of the one-launch
-    short-context path (<= 40 pages) and the split + combine pair, two layers"""
+    short-context path (<= 24 pages) and the split + combine pair, two layers"""
     nova = nova7
     print("[case] graph reference call pattern", flush=True)
     n_keys = np.array([1, 17, 640, 641, 1500], np.int32)      # 1, 2, 40, 41, 94 pages
