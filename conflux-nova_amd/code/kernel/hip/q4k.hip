@@ -58,6 +58,8 @@ constexpr int kNibWords = 32 / kLps;           // nibble dwords per lane
 struct Nib {
     uint32_t w[kNibWords];
 };
+// 16 B at any address (weights in a mapped file): one load all the same
+using u4_any __attribute__((aligned(1))) = u4;
 
 // ---------------------------------------------------------------- quant
 // One 32-element block of quant_kernel, q4k_gemv.cu:9-33: d = amax / 127,
@@ -162,7 +164,7 @@ __device__ __forceinline__ Nib load_nib(const uint8_t* blk, int c) {
     const uint8_t* p = blk + 16 + 4 * kNibWords * c;
 #pragma unroll
     for (int h = 0; h < kNibWords / 4; ++h) {
-        const u4 v = *reinterpret_cast<const u4*>(p + 16 * h);
+        const u4 v = *reinterpret_cast<const u4_any*>(p + 16 * h);
 #pragma unroll
         for (int e = 0; e < 4; ++e) n.w[4 * h + e] = v[e];
     }
@@ -347,7 +349,7 @@ __global__ void __launch_bounds__(QT) gemv_fixed_kernel(GemvSet g) {
             const int sb = kSbPerStep * t + j;
             if (sb < nsb) {
                 const uint8_t* blk = wr + (int64_t)sb * kBlockBytes;
-                hdr[t] = *reinterpret_cast<const u4*>(blk);
+                hdr[t] = *reinterpret_cast<const u4_any*>(blk);
                 nib[t] = load_nib(blk, c);
             }
         }
@@ -403,7 +405,7 @@ __global__ void __launch_bounds__(QT) gemv_split_kernel(GemvSet g) {
                 const int sb = sb0 + kSbPerStep * t;
                 if (sb < nsb) {
                     const uint8_t* blk = wr + (int64_t)sb * kBlockBytes;
-                    hdr[t] = *reinterpret_cast<const u4*>(blk);
+                    hdr[t] = *reinterpret_cast<const u4_any*>(blk);
                     nib[t] = load_nib(blk, c);
                 }
             }
@@ -789,7 +791,7 @@ __global__ void __launch_bounds__(NT) gemv4_rows_kernel(const uint8_t* __restric
         const int sb = sb0 + kSbPerStep * t;
         if (sb >= nsb) return;
         const uint8_t* blk = w + (r < rows ? r : rows - 1) * row_bytes + (int64_t)sb * kBlockBytes;
-        hdr[t] = *reinterpret_cast<const u4*>(blk);
+        hdr[t] = *reinterpret_cast<const u4_any*>(blk);
         nib[t] = load_nib(blk, c);
     };
     int64_t r = (int64_t)blockIdx.x * RPI + wave / KS;

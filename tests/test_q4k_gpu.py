@@ -150,7 +150,7 @@ def test_gemv4_matches_single_token(rows, cols, nova7, oracle):
     x[2, :32] = 0.0
     qs, d, s = oracle.quant_q8(x)
     dw, dq, dd, ds = nova.upload(w), nova.upload(qs), nova.upload(d), nova.upload(s)
-    out4 = nova.upload(np.full(4 * rows, np.nan, np.float32))
+    out4 = nova.upload(np.full(4 * rows + 64, np.nan, np.float32))      # 64 words past the output: left as they are
     nova.launch_gemv4_q4k(dw.ptr, rows, cols, dq.ptr, dd.ptr, ds.ptr, out4.ptr, None)
     singles = []
     for t in range(4):
@@ -159,7 +159,9 @@ def test_gemv4_matches_single_token(rows, cols, nova7, oracle):
                              ds.ptr + t * (cols // 16) * 4, o1.ptr, None)
         singles.append(o1)
     nova.dev_sync()
-    got = out4.numpy((4, rows), np.float32)
+    whole = out4.numpy((4 * rows + 64,), np.float32)
+    assert np.all(np.isnan(whole[4 * rows:])), "written past the output"
+    got = whole[:4 * rows].reshape(4, rows)
     # every row up to 600, else ~300 spread rows and the last 17 (a ragged last 16-row block)
     check = np.arange(rows) if rows <= 600 else np.unique(np.r_[np.arange(0, rows, rows // 300), np.arange(rows - 17, rows)])
     for t in range(4):
@@ -280,3 +282,30 @@ def test_gemv4_few_long_rows(rows, cols, nova7, oracle):
     blocks (33 super-blocks, 1024 rows on 256 CUs) and of its changes of waves
     per row, against the oracle and the one-token kernel."""
     test_gemv4_matches_single_token(rows, cols, nova7, oracle)
+
+
+@pytest.mark.parametrize("shift", [1, 2, 6])
+@pytest.mark.parametrize("rows,cols", [(37, 256), (50, 5120), (33, 13824), (20, 18944)])
+def test_gemv_weights_at_any_byte(rows, cols, shift, nova7, oracle):
+    """The one-token entry points over weights at any byte: the bits of the same
+    weights on 16 B."""
+    import ctypes as C
+    nova = nova7
+    print(f"[case] gemv rows={rows} cols={cols} weights + {shift} B", flush=True)
+    rng = np.random.default_rng(rows + cols + shift)
+    w = np.ascontiguousarray(random_blocks(rng, rows, cols)).view(np.uint8).ravel()
+    x = rng.standard_normal((1, cols)).astype(np.float32)
+    dx = nova.upload(x)
+    dq, dd, ds = (nova.upload(a) for a in oracle.quant_q8(x))
+    got = []
+    for off in (0, shift):
+        dw = nova.upload(np.concatenate([np.zeros(off, np.uint8), w]))
+        out, out32 = (nova.upload(np.full(rows, np.nan, np.float32)) for _ in range(2))
+        nova.launch_gemv_q4k(dw.ptr + off, rows, cols, dq.ptr, dd.ptr, ds.ptr, out.ptr, None)
+        nova.launch_gemv_q4k_f32((C.c_void_p * 1)(dw.ptr + off), (C.c_int64 * 1)(rows), (C.c_void_p * 1)(out32.ptr),
+                                 1, cols, dx.ptr, None)
+        nova.dev_sync()
+        got.append([o.numpy((rows,), np.uint32) for o in (out, out32)])
+    assert np.isfinite(got[0][0].view(np.float32)).all()
+    for a, b in zip(*got):
+        assert np.array_equal(a, b)
