@@ -488,14 +488,24 @@ def test_decode_single_page_ranges(model, n_keys, oracle):
     q = fx.rng.standard_normal((nova.nh, nova.hd)).astype(np.float32)
     got = _decode_single(nova, fx, q, table, n_keys)
     err64 = float(np.abs(got - _decode_f64(q, fx.hk, fx.hv, table, n_keys, nova.group)).max())
-    assert err64 < 1e-4   # 2^-22 per operand over |v| < 6, with room for fp32 sums of 32225 terms
+    print(f"  unit scale: {err64:.2e}")
+    # 2^-22 per operand of unit scale and fp32 sums: 1.3e-7 measured.  Without the
+    # lo terms of q and p it would be 1e-5 (32225 keys) to 7e-5 (641).
+    assert err64 < 1e-6
+    # queries of several units: scores up to about 30, each off by 2^-21 of itself
+    # in the exponent: 1.5e-5 of a value at worst, 5e-6 measured (fp16 queries: 1e-2)
+    q *= 6
+    got = _decode_single(nova, fx, q, table, n_keys)
+    err64 = float(np.abs(got - _decode_f64(q, fx.hk, fx.hv, table, n_keys, nova.group)).max())
+    print(f"  sharp: {err64:.2e}")
+    assert err64 < 2e-5
 
 
 @pytest.mark.parametrize("model", ["qwen25_7b", "qwen25_1p5b", "qwen25_14b"])
 def test_decode_batch_long_ranges(model, oracle):
     """More sessions than workgroups, so each has one: page ranges of 65 to 70
-    pages, past the 64 table entries of a plan record, with 1 to 8 pairs left
-    for a wave's last round."""
+    pages (33 to 35 pairs), past the 64 table entries of a plan record and not
+    whole rounds of the waves."""
     import nova_amd
     nova = nova_amd.load(model)
     n, pages = 300, 70
@@ -507,7 +517,8 @@ def test_decode_batch_long_ranges(model, oracle):
     got = _batch(nova, fx, q, tables, n_keys)
     for i in range(0, n, 13):
         ref = _decode_f64(q[i], fx.hk, fx.hv, tables[i], n_keys[i], nova.group)
-        assert np.abs(got[i] - ref).max() < 1e-4, f"session {i} n_keys={n_keys[i]}"
+        # as above; 5e-5 without the lo terms of q and p at this length
+        assert np.abs(got[i] - ref).max() < 1e-6, f"session {i} n_keys={n_keys[i]}"
 
 
 @pytest.mark.parametrize("model", ["qwen25_7b", "qwen25_1p5b", "qwen25_14b"])
@@ -529,4 +540,4 @@ def test_decode_combine_rounds(model, pages):
     got = _batch(nova, fx, q, tables, n_keys)
     for i, n in enumerate(n_keys):
         err = np.abs(got[i] - _decode_f64(q[i], fx.hk, fx.hv, tables[i], int(n), nova.group)).max()
-        assert err < 3e-6, f"{n} keys: {err:.2e}"      # operands to 2^-22, fp32 sums; 1e-4 would pass for fp16 queries
+        assert err < 3e-6, f"{n} keys: {err:.2e}"
