@@ -205,9 +205,10 @@ __device__ __forceinline__ float swap_halves(float v) {
 // Each page is a buffer resource: the loads take the page base in SGPRs and a
 // 32-bit lane offset with a scalar one, instead of a 64-bit VGPR address per
 // load (and the solo loop's prefetch does not wait on address registers still
-// being loaded).  num_records bounds
-// every load to its page; num_records = 0 makes a load return zero without a
-// memory access (a prefetch slot with no pair left).
+// being loaded).  num_records is checked against the lane offset alone, not the
+// scalar one; what keeps a load inside its page is that the two together name
+// rows 4i + g or 4g + j below 16.  num_records = 0 makes a load return zero without a memory access
+// (a prefetch slot with no pair left).
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t page_rsrc(const char* base, int bytes) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(base), 0, bytes, 0x00020000);
 }
@@ -843,9 +844,11 @@ decode_split_kernel(DecodeArgs a) {
             // The next pair's K goes out as soon as this pair's is in LDS, its
             // V when this pair's products are done: half a pair in flight per
             // wave through the arithmetic, in no more registers (16 ragged 7B
-            // sessions, 28 layers: 793 -> 777 us; with one wave per kv head,
-            // whose 8 waves stream long ranges anyway, 676 -> 683 us on four
-            // 14B layers).  The last
+            // sessions, 28 layers: 782 us with K turned by DPP moves, 793 with K
+            // through LDS, 777 with this on top: it takes back what the way
+            // through LDS costs long ranges; with one wave per kv head, whose 8
+            // waves stream long ranges anyway, 676 -> 683 us on four 14B
+            // layers).  The last
             // pair has a body of its own: loads under a condition would turn
             // the waits at the loop's head into full drains, loads without
             // effect cost the cache a pass each.

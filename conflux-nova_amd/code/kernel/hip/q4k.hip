@@ -494,8 +494,8 @@ __device__ __forceinline__ uint32_t lds_address(const unsigned char* p) {
 // two unit buffers of LDS that belong to it alone (the next unit is on its way
 // during this one's arithmetic): direct global -> LDS loads of 16 B pieces in
 // address order.  Loaded into registers the MFMA's way, the 16 rows put every
-// lane of a load on a line of its own: 343 cache accesses per unit (counted)
-// against ~75, and the cache's one access per clock set the pace (18944 x 3584:
+// lane of a load on a line of its own: 370 cache accesses per unit (counted)
+// against 90, and the cache's one access per clock set the pace (18944 x 3584:
 // 13.1 us against 11.6).  The activations come the same way, per unit and from
 // L2: staging all four first, as a dot4 kernel and an earlier form of this one
 // did, delays every launch by a round trip and a barrier.  No barrier holds a
@@ -678,7 +678,7 @@ __global__ void __launch_bounds__(64 * kMaxKs4) gemv4_kernel(const uint8_t* __re
 // codes therefore lie in four planes per token, chunk q of every quarter
 // super-block in plane q: a read's 64 lanes take 1 KiB without bank conflicts,
 // where the one-token layout's 64 B between lanes cost this kernel half its time
-// (18944 x 3584: 22.5 us, in planes 13.9); the scale and the sum of a 32 sit
+// (18944 x 3584: 22.5 us, in planes 13.5); the scale and the sum of a 32 sit
 // side by side, one read for both sub-blocks.  A row's first loads go out before
 // the activations are staged.  The four sums of a row share their cross-lane
 // steps (wave_sums4).  Workgroups of 512 threads; with 1024, a CU holds fewer of
