@@ -271,7 +271,7 @@ def test_gemv4_few_long_rows_are_spread(rows, cols, nova7):
     print(f"[case] gemv4 few long rows rows={rows} cols={cols}", flush=True)
     on, off = _gemv_us(nova, rows, cols, [(nova.launch_gemv4_q4k, 0), (nova.launch_gemv4_q4k, 4)])
     print(f"  on 16 B {on:.2f} us, off {off:.2f} us")
-    assert on < 1.15 * off
+    assert on < 1.2 * off
 
 
 @pytest.mark.parametrize("rows,cols", [(1, 8448), (1024, 8448), (1025, 8448), (1024, 8192), (7, 12288), (1024, 12544),
